@@ -1,0 +1,77 @@
+"""The production step kernel where its bookkeeping can go wrong: waves that
+are partly or barely filled, steps around the depth of its step-sum ring,
+event rates at which particles lag behind or share passes, and table rows of
+every grouping.  FP64 against the oracle's twin on the same random numbers:
+histories identical, k and E within rounding, the per-step sums of exactly
+the particles of each step."""
+import copy
+
+import numpy as np
+import pytest
+
+from emc_models import MODELS, field_force
+from oracle import oracle_py as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(spec, n, steps, dt, ppl, spl, seed=77):
+    from viennaemc_amd import emcgpu
+    M = O.OracleModel(spec)
+    ref = M.init_philox(n, O.thermal_voltage(spec["T"]), seed)
+    ctx = emcgpu.Context(precision=emcgpu.FP64)
+    ctx.setup(0, spec)
+    ctx.resize([n])
+    ctx.set_particles(0, ref["k"], ref["E"], ref["tau"], ref["valley"], ref["sub"])
+    ctx.step(dt, steps, seed=seed, step0=3, steps_per_launch=spl, ppl=ppl)
+    force, d = field_force(spec)
+    obs = M.run_philox(ref, steps, dt, force, d, seed, step0=3)
+    got = ctx.get_particles(0)
+    assert (got["valley"] == ref["valley"]).all() and (got["sub"] == ref["sub"]).all()
+    # one rounding per drift and event accumulates like the 1e-12 of the long
+    # twin runs over 100 steps
+    k, kr = got["k"].reshape(-1, 3), ref["k"].reshape(-1, 3)
+    assert (np.linalg.norm(k - kr, axis=1) <= 1e-12 * np.linalg.norm(kr, axis=1)).all()
+    assert (np.abs(got["tau"] - ref["tau"]) <= 1e-12 * dt + 1e-12 * np.abs(ref["tau"])).all()
+    av = ctx.averages(0)
+    nv = len(spec["valleys"])
+    assert (av["occ"] == obs[:, 2, :nv]).all()
+    assert np.allclose(av["avgE"], obs[:, 0, :nv], rtol=1e-11, atol=0)
+    # velocities cancel: within rounding of the thermal ones (1e5 m/s)
+    assert np.allclose(av["avgV"], obs[:, 1, :nv], rtol=1e-9, atol=1e-6)
+    # the last step's subvalley counts are those of the final state
+    cnt = np.array([[np.sum((ref["valley"] == v) & (ref["sub"] == s)) for s in range(av["sub_occ"].shape[2])]
+                    for v in range(nv)])
+    assert (np.rint(av["sub_occ"][-1] * n) == cnt).all()
+    ctx.close()
+
+
+@pytest.mark.parametrize("ppl", [1, 2, 4, 8])
+@pytest.mark.parametrize("n", [1, 63, 65, 257, 2049])
+def test_partly_filled_waves(n, ppl):
+    _run(MODELS["two_valley"], n, 21, 2e-15, ppl, 0)
+
+
+@pytest.mark.parametrize("spl", [1, 2, 15, 16, 17, 40])
+@pytest.mark.parametrize("dt", [0.05e-15, 12e-15])
+def test_rare_and_frequent_events(dt, spl):
+    """dt = 0.05 fs: about three pending events per wave and step, so that
+    they wait for each other; 12 fs: most particles scatter, several times"""
+    _run(MODELS["si_jacoboni"], 1500, 40, dt, 4, spl)
+
+
+@pytest.mark.parametrize("nt", [1, 3, 4, 5, 8, 9, 16, 17, 32])
+def test_table_rows(nt):
+    """rows of one to eight groups, the last one full or not"""
+    spec = copy.deepcopy(MODELS["si_jacoboni"])
+    base = spec["mechs"]
+    spec["mechs"] = []
+    for j in range(nt):
+        m = dict(base[j % len(base)])
+        scale = 0.3 + 0.07 * j
+        if "sigma" in m:
+            m["sigma"] *= scale
+        else:
+            m["defpot"] *= scale
+        spec["mechs"].append(m)
+    _run(spec, 700, 30, 2e-15, 2, 16)

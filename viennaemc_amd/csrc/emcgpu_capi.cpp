@@ -34,6 +34,8 @@ template <typename R>
 hipError_t launch_rebuild(const BathStepArgs<R> &a, int n_jobs, hipStream_t st);
 hipError_t launch_rates_desc(const RateDescJob *jobs, int n_jobs, int n_levels, double dE,
                              double *out, hipStream_t st);
+template <typename R>
+int fitting_ppt(StepArgs<R> a, int ppt);
 int reduce_chunks(long long max_count, int tile_size);
 hipError_t launch_reduce(const double *partial, int n_steps, int n_tiles, int n_obs, int tile_size,
                          const long long *inst_start, const long long *inst_count, int n_inst,
@@ -507,6 +509,7 @@ emcgpu_status upload_rebuild(emcgpu_ctx *c, size_t cum_elems) {
       J.n_tables = (int)tm.size();
       J.n_levels = in.n_levels;
       J.cum_off = in.cum_off[v];
+      J.tab_off = in.tab_off[v];
       for (int t = 0; t < J.n_tables; t++) {
         const emcgpu_mech_desc &md = in.mechs[tm[t]];
         J.rate_off[t] = (long long)arena.size();
@@ -597,20 +600,25 @@ emcgpu_status upload_params(emcgpu_ctx *c, double dt_s) {
   }
   std::vector<InstDev<R>> P(c->n_inst);
   std::vector<R> cum;
+  size_t cum64_elems = 0;  // FP64 copies of the tables that are rebuilt on the GPU
   for (int i = 0; i < c->n_inst; i++) {
     const Instance &in = c->inst[i];
-    std::vector<long long> off(kMaxV, 0);
+    std::vector<long long> off(kMaxV, 0), off64(kMaxV, 0);
     if (!in.has_tables)
       continue;
     for (size_t v = 0; v < in.valleys.size(); v++) {
       off[v] = (long long)cum.size();
-      const int nt = (int)in.table_mech[v].size();
-      // device layout [level][table]
+      off64[v] = (long long)cum64_elems;
+      const int nt = (int)in.table_mech[v].size(), stride = row_stride(nt);
+      cum.resize(cum.size() + (size_t)in.n_levels * stride, (R)kRowPad);
       for (int l = 0; l < in.n_levels; l++)
         for (int j = 0; j < nt; j++)
-          cum.push_back((R)in.cum[v][(size_t)j * in.n_levels + l]);
+          put_row_entry(cum.data() + off[v] + (size_t)l * stride, nt, j,
+                        (R)in.cum[v][(size_t)j * in.n_levels + l]);
+      cum64_elems += (size_t)in.n_levels * nt;
     }
-    c->inst[i].cum_off = off;
+    c->inst[i].cum_off = off64;
+    c->inst[i].tab_off = off;
     lower_instance<R>(c, in, dt_s, P[i], off);
   }
   if (cum.empty())
@@ -628,7 +636,7 @@ emcgpu_status upload_params(emcgpu_ctx *c, double dt_s) {
                            hipMemcpyHostToDevice, c->stream));
   // the host vectors die here: wait for the copies
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  emcgpu_status st = upload_rebuild<R>(c, cum.size());
+  emcgpu_status st = upload_rebuild<R>(c, cum64_elems);
   if (st)
     return st;
   c->params_dirty = false;
@@ -694,6 +702,13 @@ void fill_common(const emcgpu_ctx *c, StepArgs<R> &a) {
   for (const auto &in : c->inst)
     for (const auto &m : in.mechs)
       a.ext_kinds |= (is_scr_kind(m.kind) || is_scr_hot_kind(m.kind)) ? 1 : 0;
+  size_t used = offsetof(InstDev<R>, mech);
+  for (const auto &in : c->inst)
+    for (size_t v = 0; v < in.table_mech.size(); v++)
+      if (!in.table_mech[v].empty())
+        used = std::max(used, offsetof(InstDev<R>, mech) +
+                                  (v * kMaxMech + in.table_mech[v].size()) * sizeof(MechDev<R>));
+  a.lds_params = (int)((used + 15) & ~size_t(15));
 }
 
 // buffers of emcgpu_step_noalloc: the per-step partials and the reduction
@@ -789,10 +804,21 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
   // positions: one per lane)
   if (c->track_pos && ppl > 1)
     return fail(c, EMCGPU_ERR_ARG, "tracked positions run one particle per lane (ppl %d)", ppl);
+  StepArgs<R> a;
+  fill_common<R>(c, a);
+  if (baths) {
+    a.tally = c->d_tally;
+    a.tally_bins = c->tally_bins;
+    a.lds_bins = c->lds_bins;
+    for (const auto &in : c->inst)
+      for (const auto &m : in.mechs)
+        if (is_scr_hot_kind(m.kind) && m.q_resolved && m.q_resolved_angle)
+          a.lds_win = std::max(a.lds_win, 2 * (in.total_bins + (int)in.baths.size()));
+  }
   const int ppt = (replay || c->track_pos) ? 1
-                  : ppl                    ? ppl
-                  : c->tuned_ppl           ? c->tuned_ppl
-                                           : default_ppt(c->precision);
+                                           : fitting_ppt(a, ppl            ? ppl
+                                                            : c->tuned_ppl ? c->tuned_ppl
+                                                                           : default_ppt(c->precision));
   const int tile_size = kTile * ppt;
   const int n_tiles = (int)(c->capacity / tile_size);
   long long max_count = 0;
@@ -838,22 +864,11 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
     c->obs_steps = s->n_steps;
   }
 
-  StepArgs<R> a;
-  fill_common<R>(c, a);
   a.n_tiles = n_tiles;
   a.key0 = (uint32_t)s->seed;
   a.key1 = (uint32_t)(s->seed >> 32);
   a.partial = d_partial;
   a.dt_s = s->dt;
-  if (baths) {
-    a.tally = c->d_tally;
-    a.tally_bins = c->tally_bins;
-    a.lds_bins = c->lds_bins;
-    for (const auto &in : c->inst)
-      for (const auto &m : in.mechs)
-        if (is_scr_hot_kind(m.kind) && m.q_resolved && m.q_resolved_angle)
-          a.lds_win = std::max(a.lds_win, 2 * (in.total_bins + (int)in.baths.size()));
-  }
   const size_t n0 = c->inst[0].count;
 
   // replay and trace buffers (instance 0)

@@ -69,6 +69,28 @@ struct MechDev {
   uint8_t final_sub[kMaxDeg][kMaxZ];
 };
 
+// A valley's normalised cumulative table on the device: one row per energy
+// level, its nt entries in groups of four and, where there are several
+// groups, before them the last entry of each group (padded to a multiple of
+// four).  An event finds its mechanism with one 4-wide load of the group ends
+// and one of the group, instead of a scan whose loads wait for each other.
+// Padding holds kRowPad, above every draw.
+constexpr double kRowPad = 2.0;
+constexpr int row_groups(int nt) { return (nt + 3) / 4; }
+constexpr int row_head(int nt) { return row_groups(nt) > 1 ? 4 * row_groups(row_groups(nt)) : 0; }
+constexpr int row_stride(int nt) { return row_head(nt) + 4 * row_groups(nt); }
+// writes entry j of a row, and the group's end with it
+template <typename R>
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+inline void put_row_entry(R *row, int nt, int j, R x) {
+  const int head = row_head(nt);
+  row[head + j] = x;
+  if (head && (j % 4 == 3 || j == nt - 1))
+    row[j / 4] = x;
+}
+
 template <typename R>
 struct InstDev {
   int n_valleys;
@@ -79,9 +101,8 @@ struct InstDev {
   R vt;     // thermal voltage [V] for initialisation
   R tau0[kMaxV];  // [fs]
   int n_tables[kMaxV];
-  long long table_off[kMaxV];  // element offset of the valley's [level][table] block
+  long long table_off[kMaxV];  // element offset of the valley's table rows (row_stride)
   ValleyDev<R> valley[kMaxV];
-  MechDev<R> mech[kMaxV][kMaxMech];  // per valley, in table order
   // phonon baths of the instance: their bins are contiguous, bath b at
   // local bin offset bath_loff[b] of the instance's block that starts at
   // global bin gbin_off
@@ -100,6 +121,9 @@ struct InstDev {
   // bulk runs with positions: the periodic box [0, box] per dimension [nm]
   // (the device's maxPos, basicBulkParticleHandler.hpp:600-613)
   R box[3];
+  // per valley, in table order; last, so that a prefix of the block holds
+  // what an instance uses (the step kernel copies it into LDS)
+  alignas(8) MechDev<R> mech[kMaxV][kMaxMech];
 };
 
 // constants of one LO phonon bath (emcPhononBath<double>)
@@ -123,7 +147,8 @@ constexpr int kRateConst = 0, kRateHotAb = 1, kRateHotEm = 2, kRateScrAb = 3, kR
 constexpr int kNConst = 0, kNMean = 1, kNWindow = 2;
 struct RebuildJob {
   int inst, valley, n_tables, n_levels;
-  long long cum_off;                // element offset in the [level][table] tables
+  long long cum_off;                // element offset in the FP64 [level][table] copy
+  long long tab_off;                // element offset of the kinematics' table rows
   int kind[kMaxMech];               // kRate*
   int bath[kMaxMech];               // global bath index (hot kinds)
   double C[kMaxMech];               // rate prefactor (hot and screened kinds)
@@ -223,7 +248,14 @@ struct StepArgs {
   int lds_bins;  // bins held in LDS per block (max over instances)
   int lds_win;   // window-sum values staged in LDS per block (max over instances)
   int ext_kinds; // some instance uses a screened Froehlich kind
+  // LDS of a block of the production kernel [bytes]: the prefix of the
+  // parameters that any instance uses, tallies and window sums, each wave's
+  // particles and sums (set by the launch)
+  int lds_params, lds_hot, lds_wave;
 };
+
+// LDS of one workgroup (160 KB per CU on gfx950)
+constexpr size_t kMaxBulkLds = 160 * 1024;
 
 // ===========================================================================
 // 2-D device simulation

@@ -69,7 +69,8 @@ struct Instance {
   bool plasma() const { return scr.mode == EMCGPU_SCREENING_PLASMA && scr.enabled; }
   // periodic bulk box [m] of tracked positions (0: none)
   double box[3] = {0, 0, 0};
-  std::vector<long long> cum_off;  // per valley: element offset of the device tables
+  std::vector<long long> cum_off;  // per valley: element offset of the FP64 table copy
+  std::vector<long long> tab_off;  // per valley: element offset of the device table rows
 };
 
 }  // namespace host

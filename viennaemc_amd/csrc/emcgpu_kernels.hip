@@ -1,14 +1,13 @@
 // emcgpu_kernels.hip -- gfx950 kernels of the EMC particle step.
 //
-// A work-item owns PPT particles of a tile of 256 * PPT and keeps them in
-// registers for all steps fused into a launch, so HBM sees the SoA state
-// once per launch.  Each step is the free-flight / scatter loop of
+// A wave owns 64 * PPT particles and keeps them in LDS for all steps fused
+// into a launch, so HBM sees the SoA state once per launch.  Each step is the free-flight / scatter loop of
 // basicBulkParticleHandler::moveParticles
 // (examples/bulkSimulation/basicBulkParticleHandler.hpp:195-221):
 //   drift min(tau, dt); while (dt - tau > 0) { scatter; tau += tau';
 //   drift min(rem, tau'); rem -= tau' }; tau -= dt
-// followed by the per-step ensemble sums (wave ballot / shuffle reductions,
-// one FP64 partial per tile per step, combined by the compensated two-pass
+// followed by the per-step ensemble sums (FP64 per lane, wave reductions,
+// one FP64 partial per wave per step, combined by the compensated two-pass
 // reduction k_reduce_chunks / k_reduce_final).
 //
 // Random numbers:
@@ -162,175 +161,377 @@ __device__ __forceinline__ void tally_flush(const InstDev<R> *P, const uint32_t 
 }
 
 // ---------------------------------------------------------------------------
-// production step kernel: PPT particles per lane
+// production step kernel
 //
-// Each lane owns PPT particles of a tile of 256*PPT (particle j of lane t is
-// tile_first + j*256 + t, so every load and store is a contiguous 256-wide
-// access).  Per step all PPT particles drift min(tau, dt); then the lane
-// works through its own pending scatter events one at a time, pulling the
-// state of the next particle that still has time left into working
-// registers.  A wavefront therefore runs the scatter body while any lane
-// has any pending event among its PPT particles, which keeps most lanes
-// busy in the body instead of ~20 % (one particle per lane at ~0.24 events
-// per step).  No barriers are involved in the event loop.
+// A wave owns 64 * PPT particles (particle j * 64 + l of wave w in a tile of
+// 256 * PPT is tile_first + j * 256 + w * 64 + l, so every load and store is
+// a contiguous 64-wide access) and keeps their state in LDS for all steps of
+// the launch.  Each step every particle drifts min(tau, dt) on its own lane.
+// A particle with time left (about a fifth of them per 1 fs step in Si) is
+// queued; the wave's 64 lanes then work on queued particles, one scatter
+// event each per pass, whichever lane the particles belong to.  A particle
+// that has a further event in the step keeps its worker lane and goes on in
+// the next step's pass, behind the others (at most kRing - 1 steps); the sums
+// of a step are complete, and written, when no particle lags behind it.  The
+// random numbers are indexed by (event, step, particle), so the order of the
+// work does not change a history.  No barriers are involved.
+//
+// Bound by vector-ALU issue.  An event loop on the lane that owns the particle
+// runs the scatter body while any lane has an event left: 3.8 passes per step
+// of 256 Si particles (50 kV/cm, 1 fs) at a quarter of the lanes, 1300 VALU
+// instructions; here 1.1 passes and 684.  10M particles FP32, 64 steps:
+// 4.55 -> 3.26 ms per launch; 4M of the two-valley model FP64 (0.03 events
+// per particle and step, a pass every sixth step), 16 steps: 0.95 -> 0.71 ms.
 // ---------------------------------------------------------------------------
-// the block's instance parameters copied into LDS: every per-lane indexed
-// read of the step (subvalley accelerations, table offsets, mechanism
-// descriptors, velocity weights) then takes a 32-bit LDS address instead of
-// a 64-bit global address computed on the vector ALU
-template <typename R>
-__device__ __forceinline__ void stage_params(InstDev<R> &dst, const InstDev<R> *src) {
-  static_assert(sizeof(InstDev<R>) % 8 == 0, "8-byte copy");
-  const unsigned long long *s = reinterpret_cast<const unsigned long long *>(src);
-  unsigned long long *d = reinterpret_cast<unsigned long long *>(&dst);
-  for (int i = threadIdx.x; i < (int)(sizeof(InstDev<R>) / 8); i += kTile)
-    d[i] = s[i];
-  __syncthreads();
+// steps that a particle may lag behind, plus one: the sums of this many
+// steps are held in LDS
+constexpr int kRing = 16;
+// a pass is run while this many particles have an event pending (a wave has
+// 64 lanes); fewer wait for the next step's
+constexpr int kPass = 40;
+constexpr uint32_t kAway = 0x80000000u;  // valley/subvalley word: not with its home lane
+
+// bytes of a wave's particles and queue; its kRing * n_obs sums follow
+template <typename R, int PPT, bool POS>
+constexpr size_t fused_state_bytes() {
+  return (size_t)64 * PPT * ((POS ? 8 : 5) * sizeof(R) + sizeof(uint32_t) + sizeof(uint16_t));
 }
 
-template <typename R, int PPT, bool HOT, bool POS>
-__global__ __launch_bounds__(kTile) void k_bulk_multi(StepArgs<R> a) {
-  extern __shared__ __attribute__((aligned(16))) uint32_t lds_tally[];
-  __shared__ InstDev<R> lds_params;
-  constexpr int TS = kTile * PPT;
+// the instance's parameters: the valleys' mechanisms come last in InstDev, so
+// a prefix holds what the instance uses
+template <typename R>
+__device__ __forceinline__ const InstDev<R> *stage_params(unsigned char *lds, const InstDev<R> *src,
+                                                          int bytes) {
+  static_assert(sizeof(InstDev<R>) % 8 == 0, "8-byte copy");
+  const unsigned long long *s = reinterpret_cast<const unsigned long long *>(src);
+  unsigned long long *d = reinterpret_cast<unsigned long long *>(lds);
+  const int n = bytes < (int)sizeof(InstDev<R>) ? bytes : (int)sizeof(InstDev<R>);
+  for (int i = threadIdx.x; i < n / 8; i += kTile)
+    d[i] = s[i];
+  __syncthreads();
+  return reinterpret_cast<const InstDev<R> *>(lds);
+}
+
+__device__ __forceinline__ int lanes_below(unsigned long long mask) {
+  return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+}
+
+// energy and velocity sums of one step over the particles in step with the
+// wave, per lane in FP64
+template <typename R, int NV>
+struct StepSums {
+  double e[NV], v[NV];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      e[k] = v[k] = 0.0;
+  }
+  // the lanes with `in` enter a particle
+  __device__ __forceinline__ void add(const StepArgs<R> &a, const InstDev<R> *P, bool in, int vv,
+                                      int ss, R kx, R ky, R kz, R E) {
+    if (in) {
+      const double de = (double)E;
+      const double dv = (double)vdir_of(P->valley[NV == 1 ? 0 : vv], ss, kx, ky, kz, E);
+#pragma unroll
+      for (int k = 0; k < NV; ++k)
+        if (NV == 1 || vv == k) {
+          e[k] += de;
+          v[k] += dv;
+        }
+    }
+  }
+  // value `lane` of the step's sums, events and real events included; the
+  // counts are kept apart
+  __device__ __forceinline__ double total(const StepArgs<R> &a, int nev, int nreal) const {
+    const int lane = threadIdx.x & 63;
+    double mine = 0.0;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      if (k < a.max_v) {
+        const double se = wave_sum(e[k]), sv = wave_sum(v[k]);
+        mine = (lane == 3 + 3 * k) ? se : mine;
+        mine = (lane == 4 + 3 * k) ? sv : mine;
+      }
+    }
+    mine = (lane == 0) ? (double)nev : mine;
+    return (lane == 1) ? (double)nreal : mine;
+  }
+};
+
+// orders the wave's LDS accesses: lanes exchange particles through it
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <typename R, int PPT, bool HOT, bool POS, int NV>
+__global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  constexpr int TS = kTile * PPT, W = 64 * PPT;
   const int tile = blockIdx.x;
   const int inst = tile_instance(a.unit_inst, tile, TS);
-  stage_params(lds_params, a.inst + inst);
-  const InstDev<R> *P = &lds_params;
+  const InstDev<R> *P = stage_params(lds, a.inst + inst, a.lds_params);
+  uint32_t *lds_tally = reinterpret_cast<uint32_t *>(lds + a.lds_params);
   if constexpr (HOT)
     tally_clear(P, lds_tally);
   const long long base = a.inst_start[inst];
   const long long count = a.inst_count[inst];
-  const long long first = (long long)tile * TS - base + threadIdx.x;  // local index, j = 0
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // local index of the wave's particle 0; particle i is (i / 64) * 256 + i % 64 further on
+  const long long first = (long long)tile * TS - base + wave * 64;
 
-  R kx[PPT], ky[PPT], kz[PPT], E[PPT], tau[PPT], rem[PPT];
-  R pos[PPT][3];  // positions (POS only; folded away otherwise)
-  int v[PPT], sub[PPT];
-  uint32_t ev[PPT];
-  bool valid[PPT];
+  unsigned char *mem = lds + a.lds_params + a.lds_hot + (size_t)wave * a.lds_wave;
+  R *const skx = reinterpret_cast<R *>(mem);
+  R *const sky = skx + W, *const skz = sky + W, *const sE = skz + W, *const stau = sE + W;
+  R *const spos = stau + W;  // [3][W], POS only
+  uint32_t *const svs = reinterpret_cast<uint32_t *>(stau + (POS ? 4 : 1) * W);
+  uint16_t *const list = reinterpret_cast<uint16_t *>(svs + W);
+  double *const ring = reinterpret_cast<double *>(list + W);
+
 #pragma unroll
   for (int j = 0; j < PPT; ++j) {
-    const long long local = first + (long long)j * kTile;
-    valid[j] = local < count;
-    kx[j] = ky[j] = kz[j] = E[j] = tau[j] = rem[j] = R(0);
-    pos[j][0] = pos[j][1] = pos[j][2] = R(0);
-    v[j] = sub[j] = 0;
-    ev[j] = 0;
-    if (valid[j]) {
+    const int i = j * 64 + lane;
+    const long long local = first + (long long)j * kTile + lane;
+    uint32_t vs = 0xFFFFFFFFu;  // no particle: away for good
+    if (local < count) {
       const long long gi = base + local;
-      kx[j] = a.kx[gi];
-      ky[j] = a.ky[gi];
-      kz[j] = a.kz[gi];
-      E[j] = a.E[gi];
-      tau[j] = a.tau[gi];
-      const uint32_t vs = a.vs[gi];
-      v[j] = (int)(vs >> 16);
-      sub[j] = (int)(vs & 0xffffu);
+      skx[i] = a.kx[gi];
+      sky[i] = a.ky[gi];
+      skz[i] = a.kz[gi];
+      sE[i] = a.E[gi];
+      stau[i] = a.tau[gi];
+      vs = a.vs[gi];
       if constexpr (POS) {
-        pos[j][0] = a.px[gi];
-        pos[j][1] = a.py[gi];
-        pos[j][2] = a.pz[gi];
+        spos[i] = a.px[gi];
+        spos[W + i] = a.py[gi];
+        spos[2 * W + i] = a.pz[gi];
       }
     }
+    svs[i] = vs;
   }
+  for (int i = lane; i < kRing * a.n_obs; i += 64)
+    ring[i] = 0.0;
+  wave_lds_fence();
+  // the particles per valley and (valley, subvalley): lane o holds count o of
+  // the layout, the ring its change in each step
+  const int sub0 = 2 + 3 * a.max_v;
+  bool counts = lane >= sub0;
+  double held = 0.0;
+  for (int k = 0; k < a.max_v; ++k) {
+    int n = 0;
+    for (int d = 0; d < a.max_deg; ++d) {
+      int c = 0;
+#pragma unroll
+      for (int j = 0; j < PPT; ++j)
+        c += (int)__popcll(__ballot(svs[j * 64 + lane] == (((uint32_t)k << 16) | (uint32_t)d)));
+      n += c;
+      held = (lane == sub0 + k * a.max_deg + d) ? (double)c : held;
+    }
+    counts = counts || lane == 2 + 3 * k;
+    held = (lane == 2 + 3 * k) ? (double)n : held;
+  }
+
   StepRng<R, 0> rng;
   rng.inst = (uint32_t)inst;
   rng.k0 = a.key0;
   rng.k1 = a.key1;
   const R dt = P->dt;
+  double *const out = a.partial + (long long)tile * kSubs + wave;
+  const long long out_stride = (long long)a.n_tiles * kSubs;
+  // the sums of step r, complete, leave the ring
+  auto retire = [&](int r) {
+    if (lane < a.n_obs) {
+      double *const q = ring + (r & (kRing - 1)) * a.n_obs + lane;
+      held = *q + (counts ? held : 0.0);
+      out[((long long)r * a.n_obs + lane) * out_stride] = held;
+      *q = 0.0;
+    }
+  };
+
+  // the worker lane's particle
+  bool busy = false;
+  R kx = 0, ky = 0, kz = 0, E = 0, tau = 0, rem = 0;
+  R pos[3] = {0, 0, 0};
+  int v = 0, sub = 0, idx = 0, at = 0;  // its index in the wave, its step
+  uint32_t ev = 0;
+  uint32_t head = 0, tail = 0;  // queue of particle indices (positions modulo W)
+  int emptied = 0;         // last step whose passes emptied the queue
+  StepSums<R, NV> sums;
 
   for (int s = 0; s < a.n_steps; ++s) {
-    rng.step = a.step0 + (uint32_t)s;
+    int nev = 0, nreal = 0;
+    sums.clear();
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
-      ev[j] = 0;
-      rem[j] = R(0);
-      if (valid[j]) {
-        drift<R, POS>(P, (dt < tau[j]) ? dt : tau[j], kx[j], ky[j], kz[j], E[j], v[j], sub[j],
-                      pos[j]);
-        rem[j] = dt - tau[j];  // std::min(tau, dt) above, then tRemaining
+      const int i = j * 64 + lane;
+      const uint32_t vs = svs[i];
+      const bool here = !(vs & kAway);
+      R x = skx[i], y = sky[i], z = skz[i], en = R(0), ta = stau[i];
+      R wp[3] = {0, 0, 0};
+      const int vv = (int)(vs >> 16), ss = (int)(vs & 0xffffu);
+      bool pend = false;
+      if (here) {
+        if constexpr (POS) {
+          wp[0] = spos[i];
+          wp[1] = spos[W + i];
+          wp[2] = spos[2 * W + i];
+        }
+        // std::min(tau, dt), then tRemaining
+        drift<R, POS>(P, (dt < ta) ? dt : ta, x, y, z, en, NV == 1 ? 0 : vv, ss, wp);
+        pend = dt - ta > R(0);
+        skx[i] = x;
+        sky[i] = y;
+        skz[i] = z;
+        sE[i] = en;
+        stau[i] = pend ? ta : ta - dt;
+        if constexpr (POS) {
+          spos[i] = wp[0];
+          spos[W + i] = wp[1];
+          spos[2 * W + i] = wp[2];
+        }
+      }
+      const unsigned long long m = __ballot(pend);
+      if (pend) {
+        svs[i] = vs | kAway;
+        list[(tail + lanes_below(m)) & (W - 1)] = (uint16_t)(i | ((s & (kRing - 1)) << 12));
+      }
+      tail += (uint32_t)__popcll(m);
+      sums.add(a, P, here && !pend, vv, ss, x, y, z, en);
+    }
+    wave_lds_fence();
+
+    const bool last = s + 1 == a.n_steps;
+    for (;;) {
+      // enough pending events for a pass, or the last step of the launch,
+      // which ends with every particle, or particles that must not lag
+      // further (the queue holds none older than the step after `emptied`)
+      const unsigned long long at_work = __ballot(busy);
+      const int waiting = (int)(tail - head);
+      if (!((int)__popcll(at_work) + waiting >= kPass || (last && (waiting > 0 || at_work)) ||
+            (waiting > 0 && s - emptied >= kRing / 2) || __ballot(busy && at + (kRing - 1) <= s)))
+        break;
+      // idle lanes take the particles at the head of the queue
+      const unsigned long long idle = __ballot(!busy);
+      const int r = lanes_below(idle);
+      if (!busy && r < waiting) {
+        const int q = list[(head + r) & (W - 1)];
+        idx = q & 0xfff;
+        at = s - ((s - (q >> 12)) & (kRing - 1));
+        kx = skx[idx];
+        ky = sky[idx];
+        kz = skz[idx];
+        E = sE[idx];
+        tau = stau[idx];
+        const uint32_t vs = svs[idx];
+        v = (int)((vs & ~kAway) >> 16);
+        sub = (int)(vs & 0xffffu);
+        if constexpr (POS) {
+          pos[0] = spos[idx];
+          pos[1] = spos[W + idx];
+          pos[2] = spos[2 * W + idx];
+        }
+        rem = dt - tau;
+        ev = 0;
+        busy = true;
+      }
+      const int n_idle = (int)__popcll(idle);
+      head += (uint32_t)(n_idle < waiting ? n_idle : waiting);
+      if (tail == head)
+        emptied = s;
+
+      // one scatter event per particle
+      int real = 0;
+      const int v0 = v, sub00 = sub;
+      if (busy) {
+        rng.step = a.step0 + (uint32_t)at;
+        rng.pid = (uint32_t)(first + (long long)(idx >> 6) * kTile + (idx & 63));
+        event_once<R, 0, HOT, HOT, POS>(P, a.cum, kx, ky, kz, E, tau, rem, v, sub, ev, rng, real,
+                                        lds_tally, pos);
+      }
+      nev += (int)__popcll(__ballot(busy && at == s));
+      nreal += (int)__popcll(__ballot(real && at == s));
+      double *q = ring + (at & (kRing - 1)) * a.n_obs;
+      if (busy && at < s) {
+        atomicAdd(q, 1.0);
+        if (real)
+          atomicAdd(q + 1, 1.0);
+      }
+      if (v != v0 || sub != sub00) {
+        atomicAdd(q + sub0 + v0 * a.max_deg + sub00, -1.0);
+        atomicAdd(q + sub0 + v * a.max_deg + sub, 1.0);
+        if (NV > 1 && v != v0) {
+          atomicAdd(q + 2 + 3 * v0, -1.0);
+          atomicAdd(q + 2 + 3 * v, 1.0);
+        }
+      }
+      // particles at the end of their step: those of this step go home, those
+      // behind enter their step's sums and start the next one
+      for (;;) {
+        const bool done = busy && (!(rem > R(0)) || ev >= kMaxEventsPerStep);
+        const bool home = done && at == s, next = done && at < s;
+        if (__ballot(home)) {
+          if (home) {
+            skx[idx] = kx;
+            sky[idx] = ky;
+            skz[idx] = kz;
+            sE[idx] = E;
+            stau[idx] = tau - dt;
+            svs[idx] = ((uint32_t)v << 16) | (uint32_t)sub;
+            if constexpr (POS) {
+              spos[idx] = pos[0];
+              spos[W + idx] = pos[1];
+              spos[2 * W + idx] = pos[2];
+            }
+            busy = false;
+          }
+          sums.add(a, P, home, v, sub, kx, ky, kz, E);
+        }
+        if (!__ballot(next))
+          break;
+        if (next) {
+          q = ring + (at & (kRing - 1)) * a.n_obs;
+          atomicAdd(q + 3 + 3 * v, (double)E);
+          atomicAdd(q + 4 + 3 * v, (double)vdir_of(P->valley[NV == 1 ? 0 : v], sub, kx, ky, kz, E));
+          tau -= dt;
+          ++at;
+          ev = 0;
+          drift<R, POS>(P, (dt < tau) ? dt : tau, kx, ky, kz, E, NV == 1 ? 0 : v, sub, pos);
+          rem = dt - tau;
+        }
       }
     }
-    int nreal = 0;
-    for (;;) {
-      // next particle of this lane with time left in the step (lowest j)
-      int sel = -1;
-#pragma unroll
-      for (int j = PPT - 1; j >= 0; --j)
-        if (valid[j] && rem[j] > R(0) && ev[j] < kMaxEventsPerStep)
-          sel = j;
-      if (sel < 0)
-        break;
-      R x = kx[0], y = ky[0], z = kz[0], en = E[0], ta = tau[0], rm = rem[0];
-      R wp[3] = {pos[0][0], pos[0][1], pos[0][2]};
-      int vv = v[0], ss = sub[0];
-      uint32_t ee = ev[0];
-#pragma unroll
-      for (int j = 1; j < PPT; ++j)
-        if (sel == j) {
-          x = kx[j];
-          y = ky[j];
-          z = kz[j];
-          en = E[j];
-          ta = tau[j];
-          rm = rem[j];
-          vv = v[j];
-          ss = sub[j];
-          ee = ev[j];
-          if constexpr (POS) {
-            wp[0] = pos[j][0];
-            wp[1] = pos[j][1];
-            wp[2] = pos[j][2];
-          }
-        }
-      rng.pid = (uint32_t)(first + (long long)sel * kTile);
-      event_once<R, 0, HOT, HOT, POS>(P, a.cum, x, y, z, en, ta, rm, vv, ss, ee, rng, nreal,
-                                      lds_tally, wp);
-#pragma unroll
-      for (int j = 0; j < PPT; ++j)
-        if (sel == j) {
-          kx[j] = x;
-          ky[j] = y;
-          kz[j] = z;
-          E[j] = en;
-          tau[j] = ta;
-          rem[j] = rm;
-          v[j] = vv;
-          sub[j] = ss;
-          ev[j] = ee;
-          if constexpr (POS) {
-            pos[j][0] = wp[0];
-            pos[j][1] = wp[1];
-            pos[j][2] = wp[2];
-          }
-        }
-    }
-    int nev = 0;
-#pragma unroll
-    for (int j = 0; j < PPT; ++j) {
-      nev += (int)ev[j];
-      if (valid[j])
-        tau[j] -= dt;
-    }
-    tile_observables<R, PPT>(a, P, tile, s, valid, v, sub, kx, ky, kz, E, nev, nreal);
+    if (tail == head)
+      emptied = s;
+    wave_lds_fence();
+    const double mine = sums.total(a, nev, nreal);
+    if (lane < a.n_obs)
+      ring[(s & (kRing - 1)) * a.n_obs + lane] += mine;
+    wave_lds_fence();
+    if (s >= kRing - 1)
+      retire(s - (kRing - 1));
   }
+  for (int r = a.n_steps > kRing - 1 ? a.n_steps - (kRing - 1) : 0; r < a.n_steps; ++r)
+    retire(r);
   if constexpr (HOT)
     tally_flush(P, lds_tally, a.tally, a.tally_bins);
 
 #pragma unroll
   for (int j = 0; j < PPT; ++j) {
-    if (valid[j]) {
-      const long long gi = base + first + (long long)j * kTile;
-      a.kx[gi] = kx[j];
-      a.ky[gi] = ky[j];
-      a.kz[gi] = kz[j];
-      a.E[gi] = E[j];
-      a.tau[gi] = tau[j];
-      a.vs[gi] = ((uint32_t)v[j] << 16) | (uint32_t)sub[j];
+    const int i = j * 64 + lane;
+    const long long local = first + (long long)j * kTile + lane;
+    if (local < count) {
+      const long long gi = base + local;
+      a.kx[gi] = skx[i];
+      a.ky[gi] = sky[i];
+      a.kz[gi] = skz[i];
+      a.E[gi] = sE[i];
+      a.tau[gi] = stau[i];
+      a.vs[gi] = svs[i];
       if constexpr (POS) {
-        a.px[gi] = pos[j][0];
-        a.py[gi] = pos[j][1];
-        a.pz[gi] = pos[j][2];
+        a.px[gi] = spos[i];
+        a.py[gi] = spos[W + i];
+        a.pz[gi] = spos[2 * W + i];
       }
     }
   }
@@ -864,7 +1065,7 @@ __device__ void rebuild_one(const RebuildJob &J, const BathStepArgs<R> &a, doubl
     for (int j = 0; j < nt; ++j) {
       const long long e = J.cum_off + (long long)l * nt + j;
       const double x = cum64[e] / mx;
-      cum[e] = (R)x;
+      put_row_entry(cum + J.tab_off + (long long)l * row_stride(nt), nt, j, (R)x);
       cum64[e] = x;
     }
   }
@@ -1071,7 +1272,7 @@ __global__ __launch_bounds__(kRebuildChunk) void k_rebuild_norm(BathStepArgs<R> 
     for (int j = 0; j < nt; ++j) {
       const long long e = J.cum_off + (long long)l * nt + j;
       const double x = a.cum64[e] / mx;
-      a.cum[e] = (R)x;
+      put_row_entry(a.cum + J.tab_off + (long long)l * row_stride(nt), nt, j, (R)x);
       a.cum64[e] = x;
     }
   }
@@ -1212,52 +1413,91 @@ __global__ __launch_bounds__(kTile) void k_init_thermal(StepArgs<R> a, double in
 // particles per tile of a step-kernel variant (1 = replay / one per lane)
 int tile_size_of(int ppt) { return kTile * ppt; }
 
+// the extended kernels: bath tallies and the screened final states
+template <typename R>
+bool extended(const StepArgs<R> &a) {
+  return (a.tally && a.lds_bins > 0) || a.ext_kinds;
+}
+
+// LDS of a block of the production kernel: the parameters, tallies and
+// (8-byte aligned) staged window sums, then per wave the particles, the queue
+// and the step sums
+template <typename R, int PPT, bool POS>
+size_t fused_lds(StepArgs<R> &a) {
+  a.lds_hot = extended(a) ? (int)((sizeof(uint32_t) * 2 * (size_t)a.lds_bins + 8 +
+                                   sizeof(R) * (size_t)a.lds_win + 15) & ~size_t(15))
+                          : 0;
+  a.lds_wave = (int)((fused_state_bytes<R, PPT, POS>() +
+                      sizeof(double) * kRing * (size_t)a.n_obs + 15) & ~size_t(15));
+  return (size_t)a.lds_params + a.lds_hot + (size_t)kSubs * a.lds_wave;
+}
+
+// the particles per lane that a block's LDS holds, at most ppt
+template <typename R>
+int fitting_ppt(StepArgs<R> a, int ppt) {
+  if (ppt >= 8 && fused_lds<R, 8, false>(a) <= kMaxBulkLds)
+    return 8;
+  if (ppt >= 4 && fused_lds<R, 4, false>(a) <= kMaxBulkLds)
+    return 4;
+  if (ppt >= 2 && fused_lds<R, 2, false>(a) <= kMaxBulkLds)
+    return 2;
+  return 1;
+}
+template int fitting_ppt<float>(StepArgs<float>, int);
+template int fitting_ppt<double>(StepArgs<double>, int);
+
+template <typename R, int PPT, bool HOT, bool POS>
+hipError_t launch_fused(StepArgs<R> a, hipStream_t st) {
+  const size_t lds = fused_lds<R, PPT, POS>(a);
+  if (lds > kMaxBulkLds)
+    return hipErrorInvalidValue;
+  const void *f = a.max_v == 1 ? (const void *)k_bulk_fused<R, PPT, HOT, POS, 1>
+                               : (const void *)k_bulk_fused<R, PPT, HOT, POS, kMaxV>;
+  if (lds > 64 * 1024) {
+    const hipError_t e =
+        hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess)
+      return e;
+  }
+  void *args[] = {&a};
+  return hipLaunchKernel(f, dim3(a.n_tiles), dim3(kTile), args, lds, st);
+}
+
 template <typename R, bool HOT>
 hipError_t launch_steps_t(const StepArgs<R> &a, int mode, int ppt, hipStream_t st) {
-  const dim3 g(a.n_tiles), b(kTile);
-  // tallies, then (8-byte aligned) the staged window sums
-  const size_t lds = HOT ? sizeof(uint32_t) * 2 * (size_t)a.lds_bins + 8 +
-                               sizeof(R) * (size_t)a.lds_win
-                         : 0;
-  if (a.px) {
-    // positions tracked: one particle per lane
-    if (mode == 1)
+  if (mode == 1) {
+    // tallies, then (8-byte aligned) the staged window sums
+    const dim3 g(a.n_tiles), b(kTile);
+    const size_t lds = HOT ? sizeof(uint32_t) * 2 * (size_t)a.lds_bins + 8 +
+                                 sizeof(R) * (size_t)a.lds_win
+                           : 0;
+    if (a.px)
       hipLaunchKernelGGL((k_bulk_replay<R, HOT, true>), g, b, lds, st, a);
-    else if (ppt == 1)
-      hipLaunchKernelGGL((k_bulk_multi<R, 1, HOT, true>), g, b, lds, st, a);
     else
-      return hipErrorInvalidValue;
+      hipLaunchKernelGGL((k_bulk_replay<R, HOT, false>), g, b, lds, st, a);
     return hipGetLastError();
   }
-  if (mode == 1) {
-    hipLaunchKernelGGL((k_bulk_replay<R, HOT, false>), g, b, lds, st, a);
-  } else {
-    switch (ppt) {
-    case 1:
-      hipLaunchKernelGGL((k_bulk_multi<R, 1, HOT, false>), g, b, lds, st, a);
-      break;
-    case 2:
-      hipLaunchKernelGGL((k_bulk_multi<R, 2, HOT, false>), g, b, lds, st, a);
-      break;
-    case 4:
-      hipLaunchKernelGGL((k_bulk_multi<R, 4, HOT, false>), g, b, lds, st, a);
-      break;
-    case 8:
-      hipLaunchKernelGGL((k_bulk_multi<R, 8, HOT, false>), g, b, lds, st, a);
-      break;
-    default:
-      return hipErrorInvalidValue;
-    }
+  if (a.px)  // positions tracked: one particle per lane
+    return ppt == 1 ? launch_fused<R, 1, HOT, true>(a, st) : hipErrorInvalidValue;
+  switch (ppt) {
+  case 1:
+    return launch_fused<R, 1, HOT, false>(a, st);
+  case 2:
+    return launch_fused<R, 2, HOT, false>(a, st);
+  case 4:
+    return launch_fused<R, 4, HOT, false>(a, st);
+  case 8:
+    return launch_fused<R, 8, HOT, false>(a, st);
+  default:
+    return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
 template <typename R>
 hipError_t launch_steps(const StepArgs<R> &a, int mode, int ppt, hipStream_t st) {
   if (a.n_tiles <= 0)
     return hipSuccess;
-  // the extended kernels: bath tallies and the screened final states
-  if ((a.tally && a.lds_bins > 0) || a.ext_kinds)
+  if (extended(a))
     return launch_steps_t<R, true>(a, mode, ppt, st);
   return launch_steps_t<R, false>(a, mode, ppt, st);
 }

@@ -442,6 +442,46 @@ __device__ __forceinline__ void drift(const InstDev<R> *P, R t, R &kx, R &ky, R 
   }
 }
 
+// the table of a row (layout of row_stride) that a draw selects: the number
+// of entries <= u, i.e. the t with cum[t-1] <= u < cum[t] of the
+// non-decreasing row, -1 if u is past the last entry; lower and upper are
+// those two entries
+template <typename R>
+__device__ __forceinline__ int select_table(const R *__restrict__ row, int nt, R u, R &lower,
+                                            R &upper) {
+  typedef R Quad __attribute__((ext_vector_type(4)));
+  const Quad *q = reinterpret_cast<const Quad *>(row);
+  lower = R(0);
+  upper = R(0);
+  int g = 0;
+  const int groups = row_groups(nt);
+  if (groups > 1) {
+    for (int h = 0; h < groups; h += 4) {
+      const Quad e = *q++;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool past = e[i] <= u;
+        g += past ? 1 : 0;
+        lower = past ? e[i] : lower;
+      }
+    }
+    if (g >= groups)
+      return -1;
+  }
+  const Quad e = q[g];
+  int t = 4 * g;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const bool past = e[i] <= u;
+    t += past ? 1 : 0;
+    lower = past ? e[i] : lower;
+  }
+#pragma unroll
+  for (int i = 3; i >= 0; --i)
+    upper = (e[i] <= u) ? upper : e[i];
+  return t < nt ? t : -1;
+}
+
 // one scatter event: selection against the tables and the final state
 // (emcScatterHandler::scatterParticle, emcScatterHandler.hpp:148-170), then
 // the next free-flight time (getNewTau, emcParticleType.hpp:187-189), which
@@ -458,7 +498,6 @@ __device__ __forceinline__ R scatter_event(const InstDev<R> *P, const R *__restr
   ++e;
   if (nt > 0) {
     const int level = energy_level(P, E);
-    const R *row = cum + P->table_off[v] + (long long)level * nt;
     R usel;
     if constexpr (MODE == 0)
       usel = u[0];
@@ -466,19 +505,10 @@ __device__ __forceinline__ R scatter_event(const InstDev<R> *P, const R *__restr
       usel = (R)rng.rs.uniform(0., 1.);
     // emcScatterHandler::scatterParticle (:148-170): self scattering if
     // usel > cum[nt-1], else the first t with cum[t-1] <= usel < cum[t]
-    // (the early exit beats a branch-free count of all nt entries: most
-    // selections end in the first few, high-rate tables)
-    if (!(usel > row[nt - 1])) {
-      R lower = R(0), upper = R(0);
-      int j = -1;
-      for (int t = 0; t < nt; ++t) {
-        upper = row[t];
-        if (usel >= lower && usel < upper) {
-          j = t;
-          break;
-        }
-        lower = upper;
-      }
+    R lower, upper;
+    const int j = select_table(cum + P->table_off[v] + (long long)level * row_stride(nt), nt, usel,
+                               lower, upper);
+    {
       if (j >= 0) {
         const MechDev<R> &m = P->mech[v][j];
         R ua, ub;
