@@ -301,7 +301,7 @@ emcgpu_status emcgpu_init_particles_energy(emcgpu_ctx *ctx, int instance,
  * flight (include/emcParticleDrift.hpp:26-34) and wrapped into the device
  * box [0, maxPos] (basicBulkParticleHandler.hpp:600-613); it is written by
  * print (:227-248).  emcgpu_set_box turns this on for the context (the
- * step kernels then run one particle per lane) with the instance's box
+ * steps then take particles_per_lane 0 or 1 only) with the instance's box
  * max_pos[3] [m]; emcgpu_init_particles then also draws positions uniform
  * in the box.  Positions are [n][3] in m. */
 emcgpu_status emcgpu_set_box(emcgpu_ctx *ctx, int instance, const double max_pos[3]);

@@ -645,8 +645,17 @@ emcgpu_status upload_params(emcgpu_ctx *c, double dt_s) {
 }
 
 // particles per lane of the production kernel when the caller leaves it to
-// the library (measured best on MI355X for the Si bulk workload)
-int default_ppt(int) { return 4; }
+// the library: four (a wave's step sums and its last, partly filled passes
+// are shared by more particles; eight leave two blocks per CU), but fewer
+// where the ensemble would leave less than two waves on each of the 1024
+// SIMDs: a wave's step is then a chain of latencies that grows with its
+// particles.  Si at 50 kV/cm, us per step for 1 / 2 / 4 per lane: FP32 10k
+// 2.8 / 3.2 / 4.1, 300k 4.8 / 4.2 / 4.7, 1M 12.5 / 8.6 / 6.5; FP64 10k 4.0 /
+// 4.6 / 6.2, 300k 9.9 / 7.4 / 8.0, 1M 26.9 / 17.6 / 15.1.
+int default_ppt(const emcgpu_ctx *c) {
+  constexpr size_t kFill = 2048 * 64;
+  return c->capacity >= 4 * kFill ? 4 : c->capacity >= 2 * kFill ? 2 : 1;
+}
 
 // doubles of the per-step partials of one step (one per wave and value)
 size_t partial_per_step(const emcgpu_ctx *c, int n_tiles) {
@@ -801,7 +810,7 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
     c->bath_hist_steps = 0;
   }
   // particles per lane of the production kernel (replay and tracked
-  // positions: one per lane)
+  // positions: the caller asks for none or one per lane)
   if (c->track_pos && ppl > 1)
     return fail(c, EMCGPU_ERR_ARG, "tracked positions run one particle per lane (ppl %d)", ppl);
   StepArgs<R> a;
@@ -815,10 +824,10 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
         if (is_scr_hot_kind(m.kind) && m.q_resolved && m.q_resolved_angle)
           a.lds_win = std::max(a.lds_win, 2 * (in.total_bins + (int)in.baths.size()));
   }
-  const int ppt = (replay || c->track_pos) ? 1
-                                           : fitting_ppt(a, ppl            ? ppl
-                                                            : c->tuned_ppl ? c->tuned_ppl
-                                                                           : default_ppt(c->precision));
+  const int ppt = replay ? 1
+                         : fitting_ppt(a, ppl            ? ppl
+                                          : c->tuned_ppl ? c->tuned_ppl
+                                                         : default_ppt(c));
   const int tile_size = kTile * ppt;
   const int n_tiles = (int)(c->capacity / tile_size);
   long long max_count = 0;

@@ -1433,15 +1433,19 @@ size_t fused_lds(StepArgs<R> &a) {
 }
 
 // the particles per lane that a block's LDS holds, at most ppt
-template <typename R>
-int fitting_ppt(StepArgs<R> a, int ppt) {
-  if (ppt >= 8 && fused_lds<R, 8, false>(a) <= kMaxBulkLds)
+template <typename R, bool POS>
+int fitting_ppt_t(StepArgs<R> a, int ppt) {
+  if (!POS && ppt >= 8 && fused_lds<R, 8, POS>(a) <= kMaxBulkLds)
     return 8;
-  if (ppt >= 4 && fused_lds<R, 4, false>(a) <= kMaxBulkLds)
+  if (ppt >= 4 && fused_lds<R, 4, POS>(a) <= kMaxBulkLds)
     return 4;
-  if (ppt >= 2 && fused_lds<R, 2, false>(a) <= kMaxBulkLds)
+  if (ppt >= 2 && fused_lds<R, 2, POS>(a) <= kMaxBulkLds)
     return 2;
   return 1;
+}
+template <typename R>
+int fitting_ppt(StepArgs<R> a, int ppt) {
+  return a.px ? fitting_ppt_t<R, true>(a, ppt) : fitting_ppt_t<R, false>(a, ppt);
 }
 template int fitting_ppt<float>(StepArgs<float>, int);
 template int fitting_ppt<double>(StepArgs<double>, int);
@@ -1477,8 +1481,18 @@ hipError_t launch_steps_t(const StepArgs<R> &a, int mode, int ppt, hipStream_t s
       hipLaunchKernelGGL((k_bulk_replay<R, HOT, false>), g, b, lds, st, a);
     return hipGetLastError();
   }
-  if (a.px)  // positions tracked: one particle per lane
-    return ppt == 1 ? launch_fused<R, 1, HOT, true>(a, st) : hipErrorInvalidValue;
+  if (a.px) {  // positions tracked
+    switch (ppt) {
+    case 1:
+      return launch_fused<R, 1, HOT, true>(a, st);
+    case 2:
+      return launch_fused<R, 2, HOT, true>(a, st);
+    case 4:
+      return launch_fused<R, 4, HOT, true>(a, st);
+    default:
+      return hipErrorInvalidValue;
+    }
+  }
   switch (ppt) {
   case 1:
     return launch_fused<R, 1, HOT, false>(a, st);
