@@ -231,7 +231,7 @@ void lower_instance(const emcgpu_ctx *c, const Instance &in, double dt_s, InstDe
     }
     for (int j = 0; j < P.n_tables[v]; j++) {
       const emcgpu_mech_desc &md = in.mechs[in.table_mech[v][j]];
-      MechDev<R> &mm = P.mech[v][j];
+      MechDev<R> &mm = P.valley[v].mech[j];
       mm.final_valley = v;
       mm.z = 1;
       switch (md.kind) {
@@ -601,6 +601,11 @@ emcgpu_status upload_params(emcgpu_ctx *c, double dt_s) {
   std::vector<InstDev<R>> P(c->n_inst);
   std::vector<R> cum;
   size_t cum64_elems = 0;  // FP64 copies of the tables that are rebuilt on the GPU
+  size_t total = 0;
+  for (const Instance &in : c->inst)
+    for (size_t v = 0; in.has_tables && v < in.valleys.size(); v++)
+      total += (size_t)in.n_levels * row_stride((int)in.table_mech[v].size());
+  cum.reserve(total);
   for (int i = 0; i < c->n_inst; i++) {
     const Instance &in = c->inst[i];
     std::vector<long long> off(kMaxV, 0), off64(kMaxV, 0);
@@ -609,13 +614,21 @@ emcgpu_status upload_params(emcgpu_ctx *c, double dt_s) {
     for (size_t v = 0; v < in.valleys.size(); v++) {
       off[v] = (long long)cum.size();
       off64[v] = (long long)cum64_elems;
-      const int nt = (int)in.table_mech[v].size(), stride = row_stride(nt);
-      cum.resize(cum.size() + (size_t)in.n_levels * stride, (R)kRowPad);
-      for (int l = 0; l < in.n_levels; l++)
+      const int nt = (int)in.table_mech[v].size();
+      const int head = row_head(nt), stride = row_stride(nt);
+      const size_t nl = (size_t)in.n_levels;
+      cum.resize(cum.size() + nl * stride, (R)kRowPad);
+      R *const rows = cum.data() + off[v];
+      const double *const src = in.cum[v].data();
+      for (size_t l = 0; l < nl; l++)
         for (int j = 0; j < nt; j++)
-          put_row_entry(cum.data() + off[v] + (size_t)l * stride, nt, j,
-                        (R)in.cum[v][(size_t)j * in.n_levels + l]);
-      cum64_elems += (size_t)in.n_levels * nt;
+          rows[l * stride + head + j] = (R)src[j * nl + l];
+      for (int g = 0; head && g < row_groups(nt); g++) {
+        const int end = std::min(4 * g + 3, nt - 1);
+        for (size_t l = 0; l < nl; l++)
+          rows[l * stride + g] = rows[l * stride + head + end];
+      }
+      cum64_elems += nl * nt;
     }
     c->inst[i].cum_off = off64;
     c->inst[i].tab_off = off;
@@ -711,12 +724,12 @@ void fill_common(const emcgpu_ctx *c, StepArgs<R> &a) {
   for (const auto &in : c->inst)
     for (const auto &m : in.mechs)
       a.ext_kinds |= (is_scr_kind(m.kind) || is_scr_hot_kind(m.kind)) ? 1 : 0;
-  size_t used = offsetof(InstDev<R>, mech);
+  size_t used = offsetof(InstDev<R>, valley);
   for (const auto &in : c->inst)
     for (size_t v = 0; v < in.table_mech.size(); v++)
-      if (!in.table_mech[v].empty())
-        used = std::max(used, offsetof(InstDev<R>, mech) +
-                                  (v * kMaxMech + in.table_mech[v].size()) * sizeof(MechDev<R>));
+      used = std::max(used, offsetof(InstDev<R>, valley) + v * sizeof(ValleyBlock<R>) +
+                                sizeof(ValleyBlock<R>) -
+                                (kMaxMech - in.table_mech[v].size()) * sizeof(MechDev<R>));
   a.lds_params = (int)((used + 15) & ~size_t(15));
 }
 

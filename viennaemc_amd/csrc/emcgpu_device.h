@@ -69,6 +69,12 @@ struct MechDev {
   uint8_t final_sub[kMaxDeg][kMaxZ];
 };
 
+// a valley and its mechanisms in table order
+template <typename R>
+struct ValleyBlock : ValleyDev<R> {
+  MechDev<R> mech[kMaxMech];
+};
+
 // A valley's normalised cumulative table on the device: one row per energy
 // level, its nt entries in groups of four and, where there are several
 // groups, before them the last entry of each group (padded to a multiple of
@@ -102,7 +108,6 @@ struct InstDev {
   R tau0[kMaxV];  // [fs]
   int n_tables[kMaxV];
   long long table_off[kMaxV];  // element offset of the valley's table rows (row_stride)
-  ValleyDev<R> valley[kMaxV];
   // phonon baths of the instance: their bins are contiguous, bath b at
   // local bin offset bath_loff[b] of the instance's block that starts at
   // global bin gbin_off
@@ -121,9 +126,9 @@ struct InstDev {
   // bulk runs with positions: the periodic box [0, box] per dimension [nm]
   // (the device's maxPos, basicBulkParticleHandler.hpp:600-613)
   R box[3];
-  // per valley, in table order; last, so that a prefix of the block holds
-  // what an instance uses (the step kernel copies it into LDS)
-  alignas(8) MechDev<R> mech[kMaxV][kMaxMech];
+  // last, so that a prefix of the block holds what an instance uses (the step
+  // kernel copies it into LDS)
+  alignas(8) ValleyBlock<R> valley[kMaxV];
 };
 
 // constants of one LO phonon bath (emcPhononBath<double>)

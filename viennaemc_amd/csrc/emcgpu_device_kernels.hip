@@ -138,7 +138,7 @@ __device__ __forceinline__ bool drift_dev(const InstDev<R> *P, const DevGeom<R> 
   kx += (M[0] * ax + M[1] * ay) * t;
   ky += (M[1] * ax + M[3] * ay) * t;
   kz += (M[2] * ax + M[4] * ay) * t;
-  E = energy_of(V, kx, ky, kz);
+  E = energy_of(kane_of(V), kx, ky, kz);
   // dx = hbar M (k + k0) / 2 t / m_c(E)  [nm]: cv [m/s per 1/nm] * t [fs] * 1e-6
   const R mx = (kx + kx0) * R(0.5), my = (ky + ky0) * R(0.5), mz = (kz + kz0) * R(0.5);
   const R f = Math<R>::div(V.cv * t * R(1e-6), R(1) + R(2) * V.alpha * E);
@@ -216,7 +216,7 @@ __device__ __forceinline__ bool move_dev(const InstDev<R> *P, const R *__restric
       // emcAbstractParticleHandler.hpp:244-247)
       const InstDev<R> *Pr =
           g.region ? P + g.region[pos_coord(y, g.hy) * g.nx + pos_coord(x, g.hx)] : P;
-      const R newTau = scatter_event<R, MODE>(Pr, cum, kx, ky, kz, E, v, sub, e, rng, nreal);
+      const R newTau = scatter_event<R, MODE>(Pr, KaneAny<R>{Pr}, cum, kx, ky, kz, E, v, sub, e, rng, nreal);
       tau += newTau;
       interp(g, acc, x, y, ax, ay);
       removed = drift_dev(P, g, (newTau < rem) ? newTau : rem, ax, ay, x, y, kx, ky, kz, E, v,
@@ -259,7 +259,7 @@ __device__ __forceinline__ void new_particle(const InstDev<R> *P, const DevGeom<
   int sub = (int)Math<R>::floor((R)V.deg * (u[3] * sc + lo));
   sub = sub < V.deg ? sub : V.deg - 1;
   E = R(-1.5) * P->vt * Math<R>::log(u[4] * sc + lo);
-  random_direction(normk_of(V, E), u[5], u[6], kx, ky, kz);
+  random_direction(normk_of(kane_of(V), E), u[5], u[6], kx, ky, kz);
   if ((cx == 0 && kx < R(0)) || (cx == g.nx - 1 && kx > R(0)))
     kx = -kx;
   if ((cy == 0 && ky < R(0)) || (cy == g.ny - 1 && ky > R(0)))

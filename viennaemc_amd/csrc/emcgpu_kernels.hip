@@ -66,6 +66,36 @@ __device__ __forceinline__ int wave_sum_i(int x) {
   return __builtin_amdgcn_readlane(x, 63);
 }
 
+// the wave's sums of e and v at once: the first stage leaves each lane one of
+// them (v in the lanes whose parity is `vpar`, e in the others), the others
+// reduce lanes of one parity, so two sums cost 26 instructions instead of 40
+__device__ __forceinline__ double wave_sum_pair(double e, double v, int vpar) {
+  const bool has_v = (int)(threadIdx.x & 1u) == vpar;
+  double x = (has_v ? v : e) + dpp_d<0xb1, 0xf>(has_v ? e : v);  // with lane ^ 1
+  x = x + dpp_d<0x4e, 0xf>(x);                                   // lane ^ 2
+  x = x + dpp_d<0x124, 0xf>(x);                                  // rows rotated by 4, by 8
+  x = x + dpp_d<0x128, 0xf>(x);
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {  // across the rows of 16, then the halves
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+    const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+    unsigned long long p, q;
+    if (half == 0) {
+      const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+      const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+      p = ((unsigned long long)h[0] << 32) | l[0];
+      q = ((unsigned long long)h[1] << 32) | l[1];
+    } else {
+      const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+      const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+      p = ((unsigned long long)h[0] << 32) | l[0];
+      q = ((unsigned long long)h[1] << 32) | l[1];
+    }
+    x = __builtin_bit_cast(double, p) + __builtin_bit_cast(double, q);
+  }
+  return x;
+}
+
 constexpr int kObsMax = 2 + kMaxV * (3 + kMaxDeg);
 static_assert(kObsMax <= 64, "one lane per observable of a wave");
 
@@ -99,7 +129,9 @@ __device__ __forceinline__ void tile_observables(const StepArgs<R> &a, const Ins
       for (int j = 0; j < PPT; ++j) {
         const bool in = valid[j] && v[j] == vv;
         de += in ? (double)E[j] : 0.0;
-        dv += in ? (double)vdir_of(P->valley[vv], sub[j], kx[j], ky[j], kz[j], E[j]) : 0.0;
+        dv += in ? (double)vdir_of(kane_of(P->valley[vv]), P->valley[vv].wdir[sub[j]], kx[j], ky[j],
+                                   kz[j], E[j])
+                 : 0.0;
         cnt += (int)__popcll(__ballot(in));
       }
       se = wave_sum(de);
@@ -179,25 +211,45 @@ __device__ __forceinline__ void tally_flush(const InstDev<R> *P, const uint32_t 
 // Bound by vector-ALU issue.  An event loop on the lane that owns the particle
 // runs the scatter body while any lane has an event left: 3.8 passes per step
 // of 256 Si particles (50 kV/cm, 1 fs) at a quarter of the lanes, 1300 VALU
-// instructions; here 1.1 passes and 684.  10M particles FP32, 64 steps:
-// 4.55 -> 3.26 ms per launch; 4M of the two-valley model FP64 (0.03 events
-// per particle and step, a pass every sixth step), 16 steps: 0.95 -> 0.71 ms.
+// instructions; here 1.1 passes and 600.  10M particles FP32, 64 steps,
+// with the step sums: 4.39 -> 2.42 ms; 4M of the two-valley model FP64 (0.03
+// events per particle and step, a pass every fourth step), 16 steps: 1.12 ->
+// 0.57 ms.
 // ---------------------------------------------------------------------------
 // steps that a particle may lag behind, plus one: the sums of this many
 // steps are held in LDS
-constexpr int kRing = 16;
+constexpr int kRing = 8;
 // a pass is run while this many particles have an event pending (a wave has
-// 64 lanes); fewer wait for the next step's
-constexpr int kPass = 40;
-constexpr uint32_t kAway = 0x80000000u;  // valley/subvalley word: not with its home lane
+// 64 lanes); fewer wait for the next step's.  10M Si FP32 / 4M two-valley
+// FP64, ms: 8 pending 3.08 / 0.76, 16 2.91 / 0.69, 24 to 32 2.90 / 0.68,
+// 48 2.96 / 0.70, 64 3.59 / 0.71
+constexpr int kPass = 28;
+// valley/subvalley word in LDS: not with its home lane, in step at kAtShift
+constexpr uint32_t kAway = 0x80000000u;
+constexpr int kAtShift = 24;
+constexpr uint32_t kVsMask = 0x00FFFFFFu;
+static_assert(kMaxV <= 256 && kRing <= 128, "valley, step tag and kAway share a word");
 
-// bytes of a wave's particles and queue; its kRing * n_obs sums follow
+// a wave's particles in LDS: k, tau (and the position), the valley/subvalley
+// word, the queue's index; the energy follows from k.  Its kRing * n_obs
+// sums come after.  Less LDS is more waves: Si FP32 with the energy and a
+// ring of 16 leaves 4 blocks per CU (2.91 ms at 10M), with a ring of 8 five
+// (2.62 ms).
+template <int PPT>
+struct QueueIndex {
+  typedef uint8_t type;
+};
+template <>
+struct QueueIndex<8> {
+  typedef uint16_t type;
+};
 template <typename R, int PPT, bool POS>
 constexpr size_t fused_state_bytes() {
-  return (size_t)64 * PPT * ((POS ? 8 : 5) * sizeof(R) + sizeof(uint32_t) + sizeof(uint16_t));
+  return (size_t)64 * PPT *
+         ((POS ? 7 : 4) * sizeof(R) + sizeof(uint32_t) + sizeof(typename QueueIndex<PPT>::type));
 }
 
-// the instance's parameters: the valleys' mechanisms come last in InstDev, so
+// the instance's parameters: valleys and mechanisms come last in InstDev, so
 // a prefix holds what the instance uses
 template <typename R>
 __device__ __forceinline__ const InstDev<R> *stage_params(unsigned char *lds, const InstDev<R> *src,
@@ -227,19 +279,17 @@ struct StepSums {
     for (int k = 0; k < NV; ++k)
       e[k] = v[k] = 0.0;
   }
-  // the lanes with `in` enter a particle
-  __device__ __forceinline__ void add(const StepArgs<R> &a, const InstDev<R> *P, bool in, int vv,
-                                      int ss, R kx, R ky, R kz, R E) {
-    if (in) {
-      const double de = (double)E;
-      const double dv = (double)vdir_of(P->valley[NV == 1 ? 0 : vv], ss, kx, ky, kz, E);
+  // the active lanes enter a particle each
+  __device__ __forceinline__ void add(const InstDev<R> *P, const Kane<R> &K, int vv, int ss, R kx,
+                                      R ky, R kz, R E) {
+    const double de = (double)E;
+    const double dv = (double)vdir_of(K, P->valley[NV == 1 ? 0 : vv].wdir[ss], kx, ky, kz, E);
 #pragma unroll
-      for (int k = 0; k < NV; ++k)
-        if (NV == 1 || vv == k) {
-          e[k] += de;
-          v[k] += dv;
-        }
-    }
+    for (int k = 0; k < NV; ++k)
+      if (NV == 1 || vv == k) {
+        e[k] += de;
+        v[k] += dv;
+      }
   }
   // value `lane` of the step's sums, events and real events included; the
   // counts are kept apart
@@ -249,9 +299,8 @@ struct StepSums {
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
       if (k < a.max_v) {
-        const double se = wave_sum(e[k]), sv = wave_sum(v[k]);
-        mine = (lane == 3 + 3 * k) ? se : mine;
-        mine = (lane == 4 + 3 * k) ? sv : mine;
+        const double x = wave_sum_pair(e[k], v[k], k & 1);  // lane 3 + 3 k: e, the next: v
+        mine = (unsigned)(lane - 3 - 3 * k) < 2u ? x : mine;
       }
     }
     mine = (lane == 0) ? (double)nev : mine;
@@ -259,14 +308,37 @@ struct StepSums {
   }
 };
 
+// the lanes' common value, in scalar registers
+__device__ __forceinline__ float uniform_value(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x)));
+}
+__device__ __forceinline__ double uniform_value(double x) {
+  const long long b = __builtin_bit_cast(long long, x);
+  const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffll));
+  const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (long long)(unsigned)lo);
+}
+template <typename R, int NV>
+__device__ __forceinline__ auto kane_source(const InstDev<R> *P) {
+  if constexpr (NV == 1) {
+    const ValleyDev<R> &V = P->valley[0];
+    return KaneOne<R>{{uniform_value(V.c2), uniform_value(V.alpha), uniform_value(V.cv)}};
+  } else {
+    return KaneAny<R>{P};
+  }
+}
+
 // orders the wave's LDS accesses: lanes exchange particles through it
 __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
 
+// waves per SIMD that the registers leave room for: as many as the LDS does in
+// the large ensembles (FP64 two-valley: 173 VGPRs allow two waves, 168 three,
+// 0.68 -> 0.57 ms)
 template <typename R, int PPT, bool HOT, bool POS, int NV>
-__global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
+__global__ __launch_bounds__(kTile, PPT == 1 ? 1 : sizeof(R) == 8 ? 3 : 6) void k_bulk_fused(StepArgs<R> a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   constexpr int TS = kTile * PPT, W = 64 * PPT;
   const int tile = blockIdx.x;
@@ -283,10 +355,11 @@ __global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
 
   unsigned char *mem = lds + a.lds_params + a.lds_hot + (size_t)wave * a.lds_wave;
   R *const skx = reinterpret_cast<R *>(mem);
-  R *const sky = skx + W, *const skz = sky + W, *const sE = skz + W, *const stau = sE + W;
+  R *const sky = skx + W, *const skz = sky + W, *const stau = skz + W;
   R *const spos = stau + W;  // [3][W], POS only
   uint32_t *const svs = reinterpret_cast<uint32_t *>(stau + (POS ? 4 : 1) * W);
-  uint16_t *const list = reinterpret_cast<uint16_t *>(svs + W);
+  typedef typename QueueIndex<PPT>::type Index;
+  Index *const list = reinterpret_cast<Index *>(svs + W);
   double *const ring = reinterpret_cast<double *>(list + W);
 
 #pragma unroll
@@ -299,7 +372,6 @@ __global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
       skx[i] = a.kx[gi];
       sky[i] = a.ky[gi];
       skz[i] = a.kz[gi];
-      sE[i] = a.E[gi];
       stau[i] = a.tau[gi];
       vs = a.vs[gi];
       if constexpr (POS) {
@@ -337,6 +409,7 @@ __global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
   rng.k0 = a.key0;
   rng.k1 = a.key1;
   const R dt = P->dt;
+  const auto kane = kane_source<R, NV>(P);
   double *const out = a.partial + (long long)tile * kSubs + wave;
   const long long out_stride = (long long)a.n_tiles * kSubs;
   // the sums of step r, complete, leave the ring
@@ -378,12 +451,11 @@ __global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
           wp[2] = spos[2 * W + i];
         }
         // std::min(tau, dt), then tRemaining
-        drift<R, POS>(P, (dt < ta) ? dt : ta, x, y, z, en, NV == 1 ? 0 : vv, ss, wp);
+        drift<R, POS>(P, kane(vv), (dt < ta) ? dt : ta, x, y, z, en, NV == 1 ? 0 : vv, ss, wp);
         pend = dt - ta > R(0);
         skx[i] = x;
         sky[i] = y;
         skz[i] = z;
-        sE[i] = en;
         stau[i] = pend ? ta : ta - dt;
         if constexpr (POS) {
           spos[i] = wp[0];
@@ -393,11 +465,12 @@ __global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
       }
       const unsigned long long m = __ballot(pend);
       if (pend) {
-        svs[i] = vs | kAway;
-        list[(tail + lanes_below(m)) & (W - 1)] = (uint16_t)(i | ((s & (kRing - 1)) << 12));
+        svs[i] = vs | kAway | ((uint32_t)(s & (kRing - 1)) << kAtShift);
+        list[(tail + lanes_below(m)) & (W - 1)] = (Index)i;
       }
       tail += (uint32_t)__popcll(m);
-      sums.add(a, P, here && !pend, vv, ss, x, y, z, en);
+      if (here && !pend)
+        sums.add(P, kane(vv), vv, ss, x, y, z, en);
     }
     wave_lds_fence();
 
@@ -415,17 +488,16 @@ __global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
       const unsigned long long idle = __ballot(!busy);
       const int r = lanes_below(idle);
       if (!busy && r < waiting) {
-        const int q = list[(head + r) & (W - 1)];
-        idx = q & 0xfff;
-        at = s - ((s - (q >> 12)) & (kRing - 1));
+        idx = list[(head + r) & (W - 1)];
         kx = skx[idx];
         ky = sky[idx];
         kz = skz[idx];
-        E = sE[idx];
         tau = stau[idx];
         const uint32_t vs = svs[idx];
-        v = (int)((vs & ~kAway) >> 16);
+        at = s - ((s - (int)(vs >> kAtShift)) & (kRing - 1));
+        v = (int)((vs & kVsMask) >> 16);
         sub = (int)(vs & 0xffffu);
+        E = energy_of(kane(v), kx, ky, kz);
         if constexpr (POS) {
           pos[0] = spos[idx];
           pos[1] = spos[W + idx];
@@ -446,7 +518,7 @@ __global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
       if (busy) {
         rng.step = a.step0 + (uint32_t)at;
         rng.pid = (uint32_t)(first + (long long)(idx >> 6) * kTile + (idx & 63));
-        event_once<R, 0, HOT, HOT, POS>(P, a.cum, kx, ky, kz, E, tau, rem, v, sub, ev, rng, real,
+        event_once<R, 0, HOT, HOT, POS>(P, kane, a.cum, kx, ky, kz, E, tau, rem, v, sub, ev, rng, real,
                                         lds_tally, pos);
       }
       nev += (int)__popcll(__ballot(busy && at == s));
@@ -475,7 +547,6 @@ __global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
             skx[idx] = kx;
             sky[idx] = ky;
             skz[idx] = kz;
-            sE[idx] = E;
             stau[idx] = tau - dt;
             svs[idx] = ((uint32_t)v << 16) | (uint32_t)sub;
             if constexpr (POS) {
@@ -484,19 +555,20 @@ __global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
               spos[2 * W + idx] = pos[2];
             }
             busy = false;
+            sums.add(P, kane(v), v, sub, kx, ky, kz, E);
           }
-          sums.add(a, P, home, v, sub, kx, ky, kz, E);
         }
         if (!__ballot(next))
           break;
         if (next) {
           q = ring + (at & (kRing - 1)) * a.n_obs;
           atomicAdd(q + 3 + 3 * v, (double)E);
-          atomicAdd(q + 4 + 3 * v, (double)vdir_of(P->valley[NV == 1 ? 0 : v], sub, kx, ky, kz, E));
+          atomicAdd(q + 4 + 3 * v,
+                    (double)vdir_of(kane(v), P->valley[NV == 1 ? 0 : v].wdir[sub], kx, ky, kz, E));
           tau -= dt;
           ++at;
           ev = 0;
-          drift<R, POS>(P, (dt < tau) ? dt : tau, kx, ky, kz, E, NV == 1 ? 0 : v, sub, pos);
+          drift<R, POS>(P, kane(v), (dt < tau) ? dt : tau, kx, ky, kz, E, NV == 1 ? 0 : v, sub, pos);
           rem = dt - tau;
         }
       }
@@ -522,12 +594,14 @@ __global__ __launch_bounds__(kTile) void k_bulk_fused(StepArgs<R> a) {
     const long long local = first + (long long)j * kTile + lane;
     if (local < count) {
       const long long gi = base + local;
-      a.kx[gi] = skx[i];
-      a.ky[gi] = sky[i];
-      a.kz[gi] = skz[i];
-      a.E[gi] = sE[i];
+      const R x = skx[i], y = sky[i], z = skz[i];
+      const uint32_t vs = svs[i];
+      a.kx[gi] = x;
+      a.ky[gi] = y;
+      a.kz[gi] = z;
+      a.E[gi] = energy_of(kane((int)(vs >> 16)), x, y, z);
       a.tau[gi] = stau[i];
-      a.vs[gi] = svs[i];
+      a.vs[gi] = vs;
       if constexpr (POS) {
         a.px[gi] = spos[i];
         a.py[gi] = spos[W + i];
@@ -1390,7 +1464,7 @@ __global__ __launch_bounds__(kTile) void k_init_thermal(StepArgs<R> a, double in
     E = R(-1.5) * P->vt * Math<R>::log(ue);
   }
   R kx, ky, kz;
-  random_direction(normk_of(V, E), uphi, ucos, kx, ky, kz);
+  random_direction(normk_of(kane_of(V), E), uphi, ucos, kx, ky, kz);
   a.kx[gi] = kx;
   a.ky[gi] = ky;
   a.kz[gi] = kz;

@@ -61,14 +61,22 @@ struct Math<float> {
 // Philox-4x32-10 (Salmon et al., SC'11)
 // ---------------------------------------------------------------------------
 // (the 64-bit products compile to one v_mad_u64_u32 each instead of a
-// v_mul_lo_u32 + v_mul_hi_u32 pair)
+// v_mul_lo_u32 + v_mul_hi_u32 pair, the three-way xors to one v_bitop3_b32
+// each instead of two v_xor_b32)
+__host__ __device__ inline uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
 __host__ __device__ inline void philox4x32_10(uint32_t c[4], uint32_t k0, uint32_t k1) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
     const uint64_t p0 = (uint64_t)0xD2511F53u * c[0];
     const uint64_t p1 = (uint64_t)0xCD9E8D57u * c[2];
-    const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c[1] ^ k0;
-    const uint32_t n2 = (uint32_t)(p0 >> 32) ^ c[3] ^ k1;
+    const uint32_t n0 = xor3((uint32_t)(p1 >> 32), c[1], k0);
+    const uint32_t n2 = xor3((uint32_t)(p0 >> 32), c[3], k1);
     c[0] = n0;
     c[1] = (uint32_t)p1;
     c[2] = n2;
@@ -135,26 +143,54 @@ struct ReplayStream {
 // ---------------------------------------------------------------------------
 // valley kinematics (scaled units)
 // ---------------------------------------------------------------------------
+// the constants of a valley's dispersion and velocity
+template <typename R>
+struct Kane {
+  R c2, alpha, cv;
+};
+// valley -> its constants: read from the parameter block, or, where an
+// instance has a single valley, held in registers (KaneOne) so that the
+// drifts, final states and velocities of a step need no LDS reads for them
+template <typename R>
+struct KaneAny {
+  const InstDev<R> *P;
+  __device__ __forceinline__ Kane<R> operator()(int v) const {
+    const ValleyDev<R> &V = P->valley[v];
+    return {V.c2, V.alpha, V.cv};
+  }
+};
+template <typename R>
+struct KaneOne {
+  Kane<R> k;
+  __device__ __forceinline__ Kane<R> operator()(int) const { return k; }
+};
+
 // Kane dispersion: gamma = E(1 + aE) = c2 |k|^2  ->  E = 2 gamma / (1 + sqrt(1 + 4 a gamma))
 // (emcNonParabolicAnistropValley.hpp:109-113; exact for a = 0)
 template <typename R>
-__device__ __forceinline__ R energy_of(const ValleyDev<R> &V, R kx, R ky, R kz) {
+__device__ __forceinline__ R energy_of(const Kane<R> &V, R kx, R ky, R kz) {
   const R g = V.c2 * (kx * kx + ky * ky + kz * kz);
   return Math<R>::div(R(2) * g, R(1) + Math<R>::sqrt(R(1) + R(4) * V.alpha * g));
 }
 
 template <typename R>
-__device__ __forceinline__ R normk_of(const ValleyDev<R> &V, R E) {
+__device__ __forceinline__ R normk_of(const Kane<R> &V, R E) {
   const R g = E * (R(1) + V.alpha * E);
   return Math<R>::sqrt(Math<R>::div(g, V.c2));
 }
 
+// velocity along the field of a carrier with weights w = wdir[sub]
 template <typename R>
-__device__ __forceinline__ R vdir_of(const ValleyDev<R> &V, int sub, R kx, R ky, R kz, R E) {
+__device__ __forceinline__ R vdir_of(const Kane<R> &V, const R *w, R kx, R ky, R kz, R E) {
   // sqrt(1 + 4 alpha gamma(E)) = 1 + 2 alpha E for gamma = E (1 + alpha E)
   const R npf = R(1) + R(2) * V.alpha * E;
-  const R d = kx * V.wdir[sub][0] + ky * V.wdir[sub][1] + kz * V.wdir[sub][2];
+  const R d = kx * w[0] + ky * w[1] + kz * w[2];
   return Math<R>::div(V.cv * d, npf);
+}
+
+template <typename R>
+__device__ __forceinline__ Kane<R> kane_of(const ValleyDev<R> &V) {
+  return {V.c2, V.alpha, V.cv};
 }
 
 // getEnergyLevel (emcScatterHandler.hpp:237-244): floor(E/dE) - 1 as size_t
@@ -309,20 +345,24 @@ __device__ __forceinline__ R qres_cos_theta(const R *__restrict__ w, int nb, R d
 // final state of one mechanism: ua/ub are the two final-state uniforms
 // (phi / cos-theta for isotropic kinds, exponent / phi for the Froehlich
 // kinds)
-template <typename R, bool HOT = false, bool SCR = true>
-__device__ __forceinline__ void final_state(const InstDev<R> *P, const MechDev<R> &m, R &kx,
-                                            R &ky, R &kz, R &E, int &v, int &sub, R ua, R ub,
-                                            int zidx, uint32_t *lds_tally = nullptr) {
-  if (m.final_kind == kFinalIsotropicElastic) {
-    // emcAcousticScatterMechanism.hpp:70-72
-    const R n = Math<R>::sqrt(kx * kx + ky * ky + kz * kz);
-    random_direction(n, ua, ub, kx, ky, kz);
-  } else if (m.final_kind == kFinalIsotropicInelastic) {
-    // emcZeroOrderInterValleyScatterMechanism.hpp:119-129 / :262-272
-    sub = m.final_sub[sub][zidx];
-    v = m.final_valley;
-    E += m.shift;
-    const R n = normk_of(P->valley[v], E);
+template <typename R, bool HOT = false, bool SCR = true, typename KN = KaneAny<R>>
+__device__ __forceinline__ void final_state(const InstDev<R> *P, const KN &kane,
+                                            const MechDev<R> &m, R &kx, R &ky, R &kz, R &E, int &v,
+                                            int &sub, R ua, R ub, int zidx,
+                                            uint32_t *lds_tally = nullptr) {
+  const int kind = m.final_kind;
+  if (kind == kFinalIsotropicElastic || kind == kFinalIsotropicInelastic) {
+    R n;
+    if (kind == kFinalIsotropicElastic) {
+      // emcAcousticScatterMechanism.hpp:70-72
+      n = Math<R>::sqrt(kx * kx + ky * ky + kz * kz);
+    } else {
+      // emcZeroOrderInterValleyScatterMechanism.hpp:119-129 / :262-272
+      sub = m.final_sub[sub][zidx];
+      v = m.final_valley;
+      E += m.shift;
+      n = normk_of(kane(v), E);
+    }
     random_direction(n, ua, ub, kx, ky, kz);
   } else {
     // emcFroehlichInteraction.hpp:109-128 / :183-200; the hot-phonon kinds
@@ -333,13 +373,13 @@ __device__ __forceinline__ void final_state(const InstDev<R> *P, const MechDev<R
     // the screened kinds are compiled into the kernels that may meet them
     bool screened = false;
     if constexpr (SCR)
-      screened = m.final_kind == kFinalScreenedFroehlich;
+      screened = kind == kFinalScreenedFroehlich;
     if (screened) {
       // emcScreenedFroehlichInteraction.hpp:140-152 / :198-211: kI and kF
       // are the valley's |k| before and after the energy change
-      const R ki = normk_of(P->valley[v], E);
+      const R ki = normk_of(kane(v), E);
       E += m.shift;
-      kn = normk_of(P->valley[v], E);
+      kn = normk_of(kane(v), E);
       if (m.qres) {
         // the screened hot-phonon kinds with q-resolved angle (:283-290 /
         // :358-365): q through the bath's distribution, its window sums
@@ -361,7 +401,7 @@ __device__ __forceinline__ void final_state(const InstDev<R> *P, const MechDev<R
       ct = Math<R>::div(R(1) + f - Math<R>::pow(R(1) + R(2) * f, ua), f);
       ct = (ct < R(1)) ? ct : R(1);   // std::min(1, ct)
       ct = (R(-1) < ct) ? ct : R(-1); // std::max(-1, ct)
-      kn = normk_of(P->valley[v], E);
+      kn = normk_of(kane(v), E);
     }
     direction_wrt_k(kx, ky, kz, ct, ub);
     const R kc = Math<R>::sqrt(kx * kx + ky * ky + kz * kz);
@@ -418,19 +458,19 @@ struct StepRng<R, 1> {  // replay
 // R) and wraps into the periodic box like the bulk handler's driftParticle
 // (basicBulkParticleHandler.hpp:600-613); pos[3] in nm.
 template <typename R, bool POS = false>
-__device__ __forceinline__ void drift(const InstDev<R> *P, R t, R &kx, R &ky, R &kz, R &E, int v,
-                                      int sub, R *pos = nullptr) {
+__device__ __forceinline__ void drift(const InstDev<R> *P, const Kane<R> &K, R t, R &kx, R &ky,
+                                      R &kz, R &E, int v, int sub, R *pos = nullptr) {
   const ValleyDev<R> &V = P->valley[v];
   const R kx0 = kx, ky0 = ky, kz0 = kz;
   kx += V.accel[sub][0] * t;
   ky += V.accel[sub][1] * t;
   kz += V.accel[sub][2] * t;
-  E = energy_of(V, kx, ky, kz);
+  E = energy_of(K, kx, ky, kz);
   if constexpr (POS) {
     const R *M = V.hv[sub];
     const R mx = (kx + kx0) * R(0.5), my = (ky + ky0) * R(0.5), mz = (kz + kz0) * R(0.5);
     // cv [m/s per 1/nm] * t [fs] * 1e-6 -> nm
-    const R f = Math<R>::div(V.cv * t * R(1e-6), R(1) + R(2) * V.alpha * E);
+    const R f = Math<R>::div(K.cv * t * R(1e-6), R(1) + R(2) * K.alpha * E);
     R x[3] = {pos[0] + (M[0] * mx + M[1] * my + M[2] * mz) * f,
               pos[1] + (M[1] * mx + M[3] * my + M[4] * mz) * f,
               pos[2] + (M[2] * mx + M[4] * my + M[5] * mz) * f};
@@ -486,11 +526,11 @@ __device__ __forceinline__ int select_table(const R *__restrict__ row, int nt, R
 // (emcScatterHandler::scatterParticle, emcScatterHandler.hpp:148-170), then
 // the next free-flight time (getNewTau, emcParticleType.hpp:187-189), which
 // is returned; e counts the events of the step
-template <typename R, int MODE, bool HOT = false, bool SCR = true>
-__device__ __forceinline__ R scatter_event(const InstDev<R> *P, const R *__restrict__ cum, R &kx,
-                                           R &ky, R &kz, R &E, int &v, int &sub, uint32_t &e,
-                                           StepRng<R, MODE> &rng, int &nreal,
-                                           uint32_t *lds_tally = nullptr) {
+template <typename R, int MODE, bool HOT = false, bool SCR = true, typename KN = KaneAny<R>>
+__device__ __forceinline__ R scatter_event(const InstDev<R> *P, const KN &kane,
+                                           const R *__restrict__ cum, R &kx, R &ky, R &kz, R &E,
+                                           int &v, int &sub, uint32_t &e, StepRng<R, MODE> &rng,
+                                           int &nreal, uint32_t *lds_tally = nullptr) {
   const int nt = P->n_tables[v];
   R u[4];
   if constexpr (MODE == 0)
@@ -510,7 +550,7 @@ __device__ __forceinline__ R scatter_event(const InstDev<R> *P, const R *__restr
                                lower, upper);
     {
       if (j >= 0) {
-        const MechDev<R> &m = P->mech[v][j];
+        const MechDev<R> &m = P->valley[v].mech[j];
         R ua, ub;
         int zidx = 0;
         if constexpr (MODE == 0) {
@@ -539,7 +579,7 @@ __device__ __forceinline__ R scatter_event(const InstDev<R> *P, const R *__restr
             ub = (R)rng.rs.uniform(0., 1.);
           }
         }
-        final_state<R, HOT, SCR>(P, m, kx, ky, kz, E, v, sub, ua, ub, zidx, lds_tally);
+        final_state<R, HOT, SCR>(P, kane, m, kx, ky, kz, E, v, sub, ua, ub, zidx, lds_tally);
         ++nreal;
       }
     }
@@ -558,16 +598,18 @@ __device__ __forceinline__ R scatter_event(const InstDev<R> *P, const R *__restr
 // one pass of the scatter loop of moveParticles: scatter (selection +
 // final state), draw tau', drift min(rem, tau'), rem -= tau'
 // (basicBulkParticleHandler.hpp:203-212)
-template <typename R, int MODE, bool HOT = false, bool SCR = true, bool POS = false>
-__device__ __forceinline__ void event_once(const InstDev<R> *P, const R *__restrict__ cum, R &kx,
-                                           R &ky, R &kz, R &E, R &tau, R &rem, int &v, int &sub,
-                                           uint32_t &e, StepRng<R, MODE> &rng, int &nreal,
+template <typename R, int MODE, bool HOT = false, bool SCR = true, bool POS = false,
+          typename KN = KaneAny<R>>
+__device__ __forceinline__ void event_once(const InstDev<R> *P, const KN &kane,
+                                           const R *__restrict__ cum, R &kx, R &ky, R &kz, R &E,
+                                           R &tau, R &rem, int &v, int &sub, uint32_t &e,
+                                           StepRng<R, MODE> &rng, int &nreal,
                                            uint32_t *lds_tally = nullptr, R *pos = nullptr) {
-  const R newTau =
-      scatter_event<R, MODE, HOT, SCR>(P, cum, kx, ky, kz, E, v, sub, e, rng, nreal, lds_tally);
+  const R newTau = scatter_event<R, MODE, HOT, SCR>(P, kane, cum, kx, ky, kz, E, v, sub, e, rng,
+                                                    nreal, lds_tally);
   tau += newTau;
   // std::min(rem, newTau)
-  drift<R, POS>(P, (newTau < rem) ? newTau : rem, kx, ky, kz, E, v, sub, pos);
+  drift<R, POS>(P, kane(v), (newTau < rem) ? newTau : rem, kx, ky, kz, E, v, sub, pos);
   rem -= newTau;
 }
 
@@ -579,13 +621,14 @@ __device__ __forceinline__ void move_one(const InstDev<R> *P, const R *__restric
                                          StepRng<R, MODE> &rng, int &nev, int &nreal,
                                          uint32_t *lds_tally = nullptr, R *pos = nullptr) {
   const R dt = P->dt;
-  drift<R, POS>(P, (dt < tau) ? dt : tau, kx, ky, kz, E, v, sub, pos);  // std::min(tau, dt)
+  const KaneAny<R> kane{P};
+  drift<R, POS>(P, kane(v), (dt < tau) ? dt : tau, kx, ky, kz, E, v, sub, pos);  // std::min(tau, dt)
   R rem = dt - tau;
   uint32_t e = 0;
   // every pass draws tau' > 0 (the uniform is clamped below 1), so rem
   // strictly decreases; the event cap bounds the loop regardless
   while (rem > R(0) && e < kMaxEventsPerStep)
-    event_once<R, MODE, HOT, SCR, POS>(P, cum, kx, ky, kz, E, tau, rem, v, sub, e, rng, nreal,
+    event_once<R, MODE, HOT, SCR, POS>(P, kane, cum, kx, ky, kz, E, tau, rem, v, sub, e, rng, nreal,
                                        lds_tally, pos);
   nev += (int)e;
   tau -= dt;
