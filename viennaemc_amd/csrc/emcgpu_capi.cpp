@@ -660,13 +660,15 @@ emcgpu_status upload_params(emcgpu_ctx *c, double dt_s) {
 // particles per lane of the production kernel when the caller leaves it to
 // the library: four (a wave's step sums and its last, partly filled passes
 // are shared by more particles; eight leave two blocks per CU), but fewer
-// where the ensemble would leave less than two waves on each of the 1024
+// where the ensemble would leave less than 5/4 waves on each of the 1024
 // SIMDs: a wave's step is then a chain of latencies that grows with its
 // particles.  Si at 50 kV/cm, us per step for 1 / 2 / 4 per lane: FP32 10k
-// 2.8 / 3.2 / 4.1, 300k 4.8 / 4.2 / 4.7, 1M 12.5 / 8.6 / 6.5; FP64 10k 4.0 /
-// 4.6 / 6.2, 300k 9.9 / 7.4 / 8.0, 1M 26.9 / 17.6 / 15.1.
+// 2.6 / 3.0 / 3.8, 150k 3.2 / 3.3 / 4.0, 200k 3.6 / 3.4 / 4.0, 300k 4.2 / 3.9
+// / 4.3, 400k 5.7 / 4.4 / 4.3, 1M 10.6 / 7.5 / 5.8; FP64 10k 3.4 / 4.4 / 5.7,
+// 150k 5.7 / 5.6 / 5.8, 300k 9.0 / 7.3 / 7.4, 400k 11.7 / 9.6 / 7.6, 1M 24.2 /
+// 17.2 / 12.9.
 int default_ppt(const emcgpu_ctx *c) {
-  constexpr size_t kFill = 2048 * 64;
+  constexpr size_t kFill = 1280 * 64;
   return c->capacity >= 4 * kFill ? 4 : c->capacity >= 2 * kFill ? 2 : 1;
 }
 
@@ -692,8 +694,11 @@ emcgpu_status ensure_partial(emcgpu_ctx *c, int k_steps, int n_tiles) {
 emcgpu_status ensure_obs(emcgpu_ctx *c, int n_steps) {
   size_t bytes = (size_t)c->n_inst * n_steps * c->n_obs * sizeof(double);
   if (bytes > c->obs_bytes) {
-    dfreet(c->d_obs);
-    HIPCHK(c, hipMalloc((void **)&c->d_obs, bytes));
+    // an earlier call's launches may still write the old buffer
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    hfreet(c->h_obs);
+    c->obs_bytes = 0;
+    HIPCHK(c, hipHostMalloc((void **)&c->h_obs, bytes, hipHostMallocDefault));
     c->obs_bytes = bytes;
   }
   return EMCGPU_OK;
@@ -880,7 +885,7 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
     }
     d_partial = c->d_partial;
     d_chunks = c->d_chunks;
-    d_obs = c->d_obs;
+    d_obs = c->h_obs;
     if (reserve_only)
       return EMCGPU_OK;
     c->obs_steps = s->n_steps;
@@ -1367,7 +1372,7 @@ void emcgpu_destroy(emcgpu_ctx *c) {
   dfree(c->d_cum);
   dfreet(c->d_partial);
   dfreet(c->d_chunks);
-  dfreet(c->d_obs);
+  hfreet(c->h_obs);
   dfreet(c->d_obs0);
   dfree(c->px);
   dfree(c->py);
@@ -2549,9 +2554,8 @@ emcgpu_status emcgpu_get_observables(const emcgpu_ctx *c0, int instance, double 
   if (out && c->obs_steps > 0 && c->device >= 0) {
     (void)hipSetDevice(c->device);
     const size_t m = (size_t)c->obs_steps * c->n_obs;
-    HIPCHK(c, hipMemcpyAsync(out, c->d_obs + (size_t)instance * m, m * sizeof(double),
-                             hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    std::memcpy(out, c->h_obs + (size_t)instance * m, m * sizeof(double));
   }
   return EMCGPU_OK;
 }

@@ -105,7 +105,10 @@ struct emcgpu_ctx {
   size_t partial_bytes = 0;
   double *d_chunks = nullptr;  // (sum, compensation) pairs of the first reduction pass
   size_t chunk_bytes = 0;
-  double *d_obs = nullptr;
+  // per-step sums of the last call [instance][step][value], in pinned host
+  // memory that the reduction kernels write: a read waits for the stream and
+  // copies nothing from the device
+  double *h_obs = nullptr;
   size_t obs_bytes = 0;
   int obs_steps = 0;
   // timing
@@ -187,6 +190,14 @@ template <typename T>
 void dfreet(T *&p) {
   if (p) {
     (void)hipFree(p);
+    p = nullptr;
+  }
+}
+
+template <typename T>
+void hfreet(T *&p) {
+  if (p) {
+    (void)hipHostFree(p);
     p = nullptr;
   }
 }

@@ -764,11 +764,16 @@ __device__ __forceinline__ void block_twosum(double *ss, double *sc) {
   }
 }
 
+// With out (an output whose partials fit one chunk) the sum is finished here:
+// the second pass would add one pair to zero.  A pass less is about 5 us of
+// every call on an ensemble of up to 2048 waves.
 __global__ __launch_bounds__(256) void k_reduce_chunks(const double *__restrict__ partial,
                                                        int n_tiles, int tile_size,
                                                        const long long *__restrict__ inst_start,
                                                        const long long *__restrict__ inst_count,
-                                                       int n_chunks, double *__restrict__ chunk_out) {
+                                                       int n_chunks, double *__restrict__ chunk_out,
+                                                       double *__restrict__ out, int n_obs,
+                                                       int out_step0, int out_total) {
   __shared__ double ss[256], sc[256];
   const int chunk = blockIdx.x, so = blockIdx.y, inst = blockIdx.z;
   // the wave partials of the instance's tiles (tiles start on instance
@@ -785,9 +790,13 @@ __global__ __launch_bounds__(256) void k_reduce_chunks(const double *__restrict_
   sc[threadIdx.x] = comp;
   block_twosum(ss, sc);
   if (threadIdx.x == 0) {
-    double *o = chunk_out + (((long long)inst * gridDim.y + so) * n_chunks + chunk) * 2;
-    o[0] = ss[0];
-    o[1] = sc[0];
+    if (out) {
+      out[((long long)inst * out_total + out_step0) * n_obs + so] = ss[0] + sc[0];
+    } else {
+      double *o = chunk_out + (((long long)inst * gridDim.y + so) * n_chunks + chunk) * 2;
+      o[0] = ss[0];
+      o[1] = sc[0];
+    }
   }
 }
 
@@ -1642,8 +1651,10 @@ hipError_t launch_reduce(const double *partial, int n_steps, int n_tiles, int n_
   if (n_steps <= 0 || n_inst <= 0)
     return hipSuccess;
   hipLaunchKernelGGL(k_reduce_chunks, dim3(n_chunks, n_steps * n_obs, n_inst), dim3(256), 0, st,
-                     partial, n_tiles, tile_size, inst_start, inst_count, n_chunks, chunk_buf);
-  hipLaunchKernelGGL(k_reduce_final, dim3(n_steps * n_obs, n_inst), dim3(256), 0, st, chunk_buf,
+                     partial, n_tiles, tile_size, inst_start, inst_count, n_chunks, chunk_buf,
+                     n_chunks == 1 ? out : nullptr, n_obs, out_step0, out_total);
+  if (n_chunks > 1)
+    hipLaunchKernelGGL(k_reduce_final, dim3(n_steps * n_obs, n_inst), dim3(256), 0, st, chunk_buf,
                      n_chunks, n_obs, out, out_step0, out_total);
   return hipGetLastError();
 }
