@@ -489,6 +489,10 @@ struct GreenArgs {
   void *force;  // the force grid (DevFieldArgs::acc), float or double [node][2] (acc_fp64)
 };
 
+// deposits of the step kernel: atomics on row 0 of dep, a block-private grid in
+// LDS in the precision of the kinematics, or in FP64
+constexpr int kDepGlobal = 0, kDepLds = 1, kDepWide = 2;
+
 // particle step of a device ensemble
 template <typename R>
 struct DevStepArgs {
@@ -506,7 +510,7 @@ struct DevStepArgs {
   uint2 *stage;           // (particle, slot << 22 | rank in segment) at segment start
   int16_t *pslot;         // [particle] ohmic slot of the position after the move, -1 if none
   int *exit_part;         // [block][contact] particles that left through each contact
-  int lds_dep;            // deposit grid in LDS (else straight to dep row 0 with atomics)
+  int lds_dep;            // kDep*: where the step kernel sums the deposits
   int move;              // 0: classify positions only (contact rule of given positions)
   // drift-velocity channel current: sum of v_x over the moved particles
   // with chan_x0 <= x <= chan_x1 [nm], one FP64 partial per block

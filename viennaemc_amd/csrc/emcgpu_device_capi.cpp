@@ -49,7 +49,7 @@ hipError_t dev_launch_compact(const DevParticles<R> &src, const DevParticles<R> 
 template <typename R>
 hipError_t dev_launch_zero_r(R *p, long long n, hipStream_t st);
 template <typename R>
-int dev_step_blocks_per_cu(size_t lds);
+int dev_step_blocks_per_cu(size_t lds, bool wide);
 hipError_t dev_launch_zero(double *p, long long n, hipStream_t st);
 hipError_t dev_launch_zero_i(int *p, long long n, hipStream_t st);
 hipError_t dev_launch_mark(DevState *state, hipStream_t st);
@@ -159,7 +159,7 @@ struct DeviceSim {
   // step kernel
   int blocks = 0, n_seg = 0;
   size_t step_lds = 0;
-  bool lds_dep = true;
+  int lds_dep = kDepLds;
   void *d_dep = nullptr;
   double *d_dpart = nullptr;
   int rows_per_chunk = 1, n_chunks = 1;
@@ -894,14 +894,20 @@ emcgpu_status upload_device(emcgpu_ctx *c, DeviceSim &d) {
   HIPCHK(c, hipMemcpy(d.d_state, &s, sizeof s, hipMemcpyHostToDevice));
   // step kernel: a block-private deposit grid when it fits the LDS (the
   // rank kernel holds the per-wave slot counts, at most 32 KB)
+  // FP64 sums for as many nodes as fit, then sums in the precision of the
+  // kinematics, then atomics on one grid in memory
+  const size_t wide_bytes = ((nn * sizeof(double)) + 15) & ~(size_t)15;
   const size_t grid_bytes = ((nn * rs) + 15) & ~(size_t)15;
-  d.lds_dep = grid_bytes <= (size_t)kDevMaxLds;
-  d.step_lds = d.lds_dep ? grid_bytes : 0;
+  d.lds_dep = wide_bytes <= (size_t)kDevMaxLds   ? kDepWide
+              : grid_bytes <= (size_t)kDevMaxLds ? kDepLds
+                                                 : kDepGlobal;
+  d.step_lds = d.lds_dep == kDepWide ? wide_bytes : d.lds_dep == kDepLds ? grid_bytes : 0;
   hipDeviceProp_t prop;
   HIPCHK(c, hipGetDeviceProperties(&prop, c->device));
   // one step block per CU (its waves share the CU's chunks)
-  const int per_cu = c->precision == EMCGPU_FP32 ? dev_step_blocks_per_cu<float>(d.step_lds)
-                                                 : dev_step_blocks_per_cu<double>(d.step_lds);
+  const bool wide = d.lds_dep == kDepWide;
+  const int per_cu = c->precision == EMCGPU_FP32 ? dev_step_blocks_per_cu<float>(d.step_lds, wide)
+                                                 : dev_step_blocks_per_cu<double>(d.step_lds, wide);
   if (per_cu < 1)
     return fail(c, EMCGPU_ERR_ARG, "the step kernel does not fit a CU");
   d.blocks = prop.multiProcessorCount;
@@ -1158,7 +1164,7 @@ DevStepArgs<R> step_args(const emcgpu_ctx *c, const DeviceSim &d) {
   a.stage = d.d_stage;
   a.pslot = d.d_pslot;
   a.exit_part = d.d_exit_part;
-  a.lds_dep = d.lds_dep ? 1 : 0;
+  a.lds_dep = d.lds_dep;
   a.move = 1;
   a.chan = d.chan;
   a.chan_x0 = (R)d.chan_x0;

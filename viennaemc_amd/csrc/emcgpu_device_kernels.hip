@@ -365,7 +365,13 @@ __device__ __forceinline__ void segment_range(long long n, long long n_seg, long
 // take more of them, and load the state of their next chunk while the
 // current one moves.  (A copy of the force grid in LDS measured slower: the
 // copy costs more than the L2 gathers it saves.)
-template <typename R>
+//
+// G is the type of the block's deposit grid in LDS: double where it fits (20k
+// nodes).  ds_add_f32 takes about 195 cycles for a wave whatever its
+// addresses, ds_add_f64 10 to 22 (66 where the lanes share four addresses),
+// and the FP64 sums lose no carriers to rounding; with FP32 sums the atomics
+// were 60 % of the kernel's time (2M particles FP32: 57 -> 38 us).
+template <typename R, typename G>
 __global__ __launch_bounds__(DevStepShape<R>::threads) void k_dev_step(DevStepArgs<R> a) {
   constexpr int NT = DevStepShape<R>::threads, NW = DevStepShape<R>::waves;
   extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -374,10 +380,10 @@ __global__ __launch_bounds__(DevStepShape<R>::threads) void k_dev_step(DevStepAr
   __shared__ int q_next;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int nn = a.g.nn;
-  R *grid = (R *)lds_raw;
+  G *grid = (G *)lds_raw;
   if (a.lds_dep)
     for (int k = tid; k < nn; k += NT)
-      grid[k] = R(0);
+      grid[k] = G(0);
   if (tid < kMaxContacts)
     ex_cnt[tid] = 0;
   if (tid == 0)
@@ -460,7 +466,7 @@ __global__ __launch_bounds__(DevStepShape<R>::threads) void k_dev_step(DevStepAr
       }
       if (!removed) {
         if (a.lds_dep)
-          assign(a.g, x, y, [&](int k, R w) { atomicAdd(&grid[k], w); });
+          assign(a.g, x, y, [&](int k, R w) { atomicAdd(&grid[k], (G)w); });
         else
           assign(a.g, x, y, [&](int k, R w) { atomicAdd(&a.dep[k], w); });
         const int cx = pos_coord(x, a.g.hx), cy = pos_coord(y, a.g.hy);
@@ -488,7 +494,7 @@ __global__ __launch_bounds__(DevStepShape<R>::threads) void k_dev_step(DevStepAr
   }
   if (a.lds_dep)
     for (int k = tid; k < nn; k += NT)
-      a.dep[(long long)blockIdx.x * nn + k] = grid[k];
+      a.dep[(long long)blockIdx.x * nn + k] = (R)grid[k];
   if (tid < a.n_contacts && a.exit_part)
     a.exit_part[blockIdx.x * a.n_contacts + tid] = ex_cnt[tid];
 }
@@ -1990,20 +1996,31 @@ hipError_t dev_launch_field(const DevFieldArgs<R> *args_dev, size_t lds, bool ws
   return hipGetLastError();
 }
 
+// the step kernel with an FP64 or an R deposit grid in LDS
+template <typename R>
+const void *dev_step_kernel(bool wide) {
+  return wide ? (const void *)k_dev_step<R, double> : (const void *)k_dev_step<R, R>;
+}
+
 template <typename R>
 hipError_t dev_launch_step(const DevStepArgs<R> &a, const DevContactArgs<R> &ca, int blocks,
                            int n_seg, size_t lds, hipStream_t st) {
   if (lds > (size_t)kDevMaxLds)
     return hipErrorInvalidValue;
+  const void *f = dev_step_kernel<R>(a.lds_dep == kDepWide);
   if (lds > 65536) {
-    hipError_t e = hipFuncSetAttribute((const void *)k_dev_step<R>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e =
+        hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) {
       (void)hipGetLastError();
       return e;
     }
   }
-  hipLaunchKernelGGL((k_dev_step<R>), dim3(blocks), dim3(DevStepShape<R>::threads), lds, st, a);
+  void *args[] = {const_cast<DevStepArgs<R> *>(&a)};
+  const hipError_t e =
+      hipLaunchKernel(f, dim3(blocks), dim3(DevStepShape<R>::threads), args, lds, st);
+  if (e != hipSuccess)
+    return e;
   const int n_rank = n_seg / kDevStepWaves;
   const int node_blocks = (ca.g.nn + kDevStepThreads - 1) / kDevStepThreads;
   hipLaunchKernelGGL((k_dev_rank_rows<R>), dim3((unsigned)(n_rank + node_blocks * ca.n_chunks)),
@@ -2067,16 +2084,15 @@ hipError_t dev_launch_mark(DevState *state, hipStream_t st) {
 
 // resident step blocks per CU at the given dynamic LDS
 template <typename R>
-int dev_step_blocks_per_cu(size_t lds) {
+int dev_step_blocks_per_cu(size_t lds, bool wide) {
   int n = 0;
-  if (lds > 65536 &&
-      hipFuncSetAttribute((const void *)k_dev_step<R>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)lds) != hipSuccess) {
+  const void *f = dev_step_kernel<R>(wide);
+  if (lds > 65536 && hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         (int)lds) != hipSuccess) {
     (void)hipGetLastError();
     return 0;
   }
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_dev_step<R>, DevStepShape<R>::threads,
-                                                   lds) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, DevStepShape<R>::threads, lds) !=
       hipSuccess)
     return 1;
   return n;
@@ -2507,7 +2523,7 @@ hipError_t dev_launch_green_expand(const double *Ainv, long long lda, const int 
   template hipError_t dev_launch_compact<R>(const DevParticles<R> &, const DevParticles<R> &, \
                                             int *, long long, DevState *, hipStream_t);       \
   template hipError_t dev_launch_zero_r<R>(R *, long long, hipStream_t);                      \
-  template int dev_step_blocks_per_cu<R>(size_t);
+  template int dev_step_blocks_per_cu<R>(size_t, bool);
 EMCGPU_DEV_INST(float)
 EMCGPU_DEV_INST(double)
 
