@@ -75,3 +75,12 @@ def test_table_rows(nt):
             m["defpot"] *= scale
         spec["mechs"].append(m)
     _run(spec, 700, 30, 2e-15, 2, 16)
+
+
+@pytest.mark.parametrize("ppl", [1, 2, 4, 8])
+@pytest.mark.parametrize("model,dt", [("screened_polar", 0.5e-15), ("two_valley", 15e-15)])
+def test_one_step_launches(model, dt, ppl):
+    """the streaming kernel of one-step launches: waves whose particles come
+    in one to eight chunks of 64, the last one ragged, with few and with
+    mostly scattering particles"""
+    _run(MODELS[model], 1801, 12, dt, ppl, 1)

@@ -666,9 +666,12 @@ emcgpu_status upload_params(emcgpu_ctx *c, double dt_s) {
 // 2.6 / 3.0 / 3.8, 150k 3.2 / 3.3 / 4.0, 200k 3.6 / 3.4 / 4.0, 300k 4.2 / 3.9
 // / 4.3, 400k 5.7 / 4.4 / 4.3, 1M 10.6 / 7.5 / 5.8; FP64 10k 3.4 / 4.4 / 5.7,
 // 150k 5.7 / 5.6 / 5.8, 300k 9.0 / 7.3 / 7.4, 400k 11.7 / 9.6 / 7.6, 1M 24.2 /
-// 17.2 / 12.9.
-int default_ppt(const emcgpu_ctx *c) {
-  constexpr size_t kFill = 1280 * 64;
+// 17.2 / 12.9.  One-step launches in FP64 stream their particles and take
+// eight per lane (screened cooling, 1M: 51.7 us with four, 41.8 with eight).
+int default_ppt(const emcgpu_ctx *c, bool one_step) {
+  constexpr long long kFill = 1280 * 64;
+  if (one_step && c->precision == EMCGPU_FP64 && c->capacity >= 8 * kFill)
+    return 8;
   return c->capacity >= 4 * kFill ? 4 : c->capacity >= 2 * kFill ? 2 : 1;
 }
 
@@ -677,7 +680,10 @@ size_t partial_per_step(const emcgpu_ctx *c, int n_tiles) {
   return (size_t)std::max(n_tiles, 1) * kSubs * (size_t)c->n_obs;
 }
 // doubles of the first reduction pass's (sum, compensation) pairs per step
+// (one chunk: summed to the end in one pass)
 size_t chunks_per_step(const emcgpu_ctx *c, int n_chunks) {
+  if (n_chunks == 1)
+    return 0;
   return (size_t)c->n_inst * (size_t)c->n_obs * (size_t)n_chunks * 2;
 }
 
@@ -845,7 +851,7 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
   const int ppt = replay ? 1
                          : fitting_ppt(a, ppl            ? ppl
                                           : c->tuned_ppl ? c->tuned_ppl
-                                                         : default_ppt(c));
+                                                         : default_ppt(c, K == 1));
   const int tile_size = kTile * ppt;
   const int n_tiles = (int)(c->capacity / tile_size);
   long long max_count = 0;

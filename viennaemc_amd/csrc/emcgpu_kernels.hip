@@ -612,6 +612,228 @@ __global__ __launch_bounds__(kTile, PPT == 1 ? 1 : sizeof(R) == 8 ? 3 : 6) void 
 }
 
 // ---------------------------------------------------------------------------
+// production step kernel of launches with one step (phonon baths and plasma
+// screening, and callers that step one at a time): the particles stream
+// through, 64 of the wave's 64 * PPT at a time with the next 64 on their way;
+// those without an event are done after their flight, the others wait in LDS
+// until a pass fills the wave's lanes.  Only a wave's last passes are partly
+// filled, so more particles per lane mean fewer idle lanes, and the particles
+// take no LDS.  Used in FP64, whose scatter body is long (screened cooling
+// with 0.13 events per particle and step, 1M: 53.6 -> 41.8 us per step with
+// 8 per lane, 4M: 134.7 -> 106.6), and for small ensembles (50k FP32: 11.9 ->
+// 10.8).  In FP32 the stores of single particles cost more than the passes
+// they save (4M Si: 47.4 us with the particles in LDS, 55.5 streamed).
+// ---------------------------------------------------------------------------
+template <typename R>
+constexpr bool streams_one_step(int ppt) {
+  return sizeof(R) == 8 || ppt <= 2;
+}
+// queue entries of a wave: less than a pass's worth waits when 64 more arrive
+constexpr int kOnceQueue = 128;
+constexpr int kOncePass = 60;  // pending events that make a pass worth its while
+
+template <typename R, bool POS>
+constexpr size_t once_wave_bytes() {
+  return (size_t)kOnceQueue * ((POS ? 7 : 4) * sizeof(R) + sizeof(uint32_t) + sizeof(uint16_t));
+}
+
+template <typename R, int PPT, bool HOT, bool POS, int NV>
+__global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(StepArgs<R> a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  constexpr int TS = kTile * PPT, Q = kOnceQueue;
+  const int tile = blockIdx.x;
+  const int inst = tile_instance(a.unit_inst, tile, TS);
+  const InstDev<R> *P = stage_params(lds, a.inst + inst, a.lds_params);
+  uint32_t *lds_tally = reinterpret_cast<uint32_t *>(lds + a.lds_params);
+  if constexpr (HOT)
+    tally_clear(P, lds_tally);
+  const long long base = a.inst_start[inst];
+  const long long count = a.inst_count[inst];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // local index of the wave's particle 0; particle i is (i / 64) * 256 + i % 64 further on
+  const long long first = (long long)tile * TS - base + wave * 64;
+
+  unsigned char *mem = lds + a.lds_params + a.lds_hot + (size_t)wave * a.lds_wave;
+  R *const qx = reinterpret_cast<R *>(mem);
+  R *const qy = qx + Q, *const qz = qy + Q, *const qtau = qz + Q, *const qpos = qtau + Q;
+  uint32_t *const qvs = reinterpret_cast<uint32_t *>(qtau + (POS ? 4 : 1) * Q);
+  uint16_t *const qidx = reinterpret_cast<uint16_t *>(qvs + Q);
+  double *const delta = reinterpret_cast<double *>(qidx + Q);  // changes of the counts [n_obs]
+  for (int i = lane; i < a.n_obs; i += 64)
+    delta[i] = 0.0;
+
+  StepRng<R, 0> rng;
+  rng.inst = (uint32_t)inst;
+  rng.step = a.step0;
+  rng.k0 = a.key0;
+  rng.k1 = a.key1;
+  const R dt = P->dt;
+  const auto kane = kane_source<R, NV>(P);
+  const int sub0 = 2 + 3 * a.max_v;
+
+  struct Part {
+    R x, y, z, tau, pos[3];
+    uint32_t vs;
+    bool valid;
+  };
+  auto load = [&](int j, Part &p) {
+    const long long local = first + (long long)j * kTile + lane;
+    p.valid = j < PPT && local < count;
+    p.vs = 0xFFFFFFFFu;
+    if (p.valid) {
+      const long long gi = base + local;
+      p.x = a.kx[gi];
+      p.y = a.ky[gi];
+      p.z = a.kz[gi];
+      p.tau = a.tau[gi];
+      p.vs = a.vs[gi];
+      if constexpr (POS) {
+        p.pos[0] = a.px[gi];
+        p.pos[1] = a.py[gi];
+        p.pos[2] = a.pz[gi];
+      }
+    }
+  };
+  auto store = [&](int i, R x, R y, R z, R E, R tau, const R *pos) {
+    const long long gi = base + first + (long long)(i >> 6) * kTile + (i & 63);
+    a.kx[gi] = x;
+    a.ky[gi] = y;
+    a.kz[gi] = z;
+    a.E[gi] = E;
+    a.tau[gi] = tau;
+    if constexpr (POS) {
+      a.px[gi] = pos[0];
+      a.py[gi] = pos[1];
+      a.pz[gi] = pos[2];
+    }
+    return gi;
+  };
+
+  // the worker lane's particle
+  bool busy = false;
+  R kx = 0, ky = 0, kz = 0, E = 0, tau = 0, rem = 0;
+  R pos[3] = {0, 0, 0};
+  int v = 0, sub = 0, idx = 0;
+  uint32_t ev = 0, head = 0, tail = 0;
+  int nev = 0, nreal = 0;
+  double held = 0.0;  // lane o: count o of the layout before the step's events
+  StepSums<R, NV> sums;
+  sums.clear();
+
+  // passes while `enough` events are pending
+  auto passes = [&](int enough) {
+    for (;;) {
+      const int waiting = (int)(tail - head);
+      if ((int)__popcll(__ballot(busy)) + waiting < enough)
+        break;
+      const unsigned long long idle = __ballot(!busy);
+      const int r = lanes_below(idle);
+      if (!busy && r < waiting) {
+        const int q = (int)((head + (uint32_t)r) & (Q - 1));
+        idx = qidx[q];
+        kx = qx[q];
+        ky = qy[q];
+        kz = qz[q];
+        tau = qtau[q];
+        const uint32_t vs = qvs[q];
+        v = (int)(vs >> 16);
+        sub = (int)(vs & 0xffffu);
+        if constexpr (POS) {
+          pos[0] = qpos[q];
+          pos[1] = qpos[Q + q];
+          pos[2] = qpos[2 * Q + q];
+        }
+        E = energy_of(kane(v), kx, ky, kz);
+        rem = dt - tau;
+        ev = 0;
+        busy = true;
+      }
+      const int n_idle = (int)__popcll(idle);
+      head += (uint32_t)(n_idle < waiting ? n_idle : waiting);
+      int real = 0;
+      const int v0 = v, sub00 = sub;
+      if (busy) {
+        rng.pid = (uint32_t)(first + (long long)(idx >> 6) * kTile + (idx & 63));
+        event_once<R, 0, HOT, HOT, POS>(P, kane, a.cum, kx, ky, kz, E, tau, rem, v, sub, ev, rng,
+                                        real, lds_tally, pos);
+      }
+      nev += (int)__popcll(__ballot(busy));
+      nreal += (int)__popcll(__ballot(real));
+      if (v != v0 || sub != sub00) {
+        atomicAdd(delta + sub0 + v0 * a.max_deg + sub00, -1.0);
+        atomicAdd(delta + sub0 + v * a.max_deg + sub, 1.0);
+        if (NV > 1 && v != v0) {
+          atomicAdd(delta + 2 + 3 * v0, -1.0);
+          atomicAdd(delta + 2 + 3 * v, 1.0);
+        }
+      }
+      if (busy && (!(rem > R(0)) || ev >= kMaxEventsPerStep)) {
+        const long long gi = store(idx, kx, ky, kz, E, tau - dt, pos);
+        a.vs[gi] = ((uint32_t)v << 16) | (uint32_t)sub;
+        sums.add(P, kane(v), v, sub, kx, ky, kz, E);
+        busy = false;
+      }
+    }
+  };
+
+  Part next;
+  load(0, next);
+#pragma unroll 1
+  for (int j = 0; j < PPT; ++j) {
+    Part p = next;
+    load(j + 1, next);
+    const int vv = (int)(p.vs >> 16), ss = (int)(p.vs & 0xffffu);
+    for (int k = 0; k < a.max_v; ++k) {
+      int n = 0;
+      for (int d = 0; d < a.max_deg; ++d) {
+        const int c = (int)__popcll(__ballot(p.valid && (NV == 1 || vv == k) && ss == d));
+        n += c;
+        held += (lane == sub0 + k * a.max_deg + d) ? (double)c : 0.0;
+      }
+      held += (lane == 2 + 3 * k) ? (double)n : 0.0;
+    }
+    bool pend = false;
+    if (p.valid) {
+      R en = R(0);
+      drift<R, POS>(P, kane(vv), (dt < p.tau) ? dt : p.tau, p.x, p.y, p.z, en, NV == 1 ? 0 : vv, ss,
+                    p.pos);
+      pend = dt - p.tau > R(0);
+      if (!pend) {
+        store(j * 64 + lane, p.x, p.y, p.z, en, p.tau - dt, p.pos);
+        sums.add(P, kane(vv), vv, ss, p.x, p.y, p.z, en);
+      }
+    }
+    const unsigned long long m = __ballot(pend);
+    if (pend) {
+      const int q = (int)((tail + (uint32_t)lanes_below(m)) & (Q - 1));
+      qx[q] = p.x;
+      qy[q] = p.y;
+      qz[q] = p.z;
+      qtau[q] = p.tau;
+      qvs[q] = p.vs;
+      qidx[q] = (uint16_t)(j * 64 + lane);
+      if constexpr (POS) {
+        qpos[q] = p.pos[0];
+        qpos[Q + q] = p.pos[1];
+        qpos[2 * Q + q] = p.pos[2];
+      }
+    }
+    tail += (uint32_t)__popcll(m);
+    wave_lds_fence();
+    passes(kOncePass);
+    wave_lds_fence();
+  }
+  passes(1);
+  wave_lds_fence();
+  const double mine = sums.total(a, nev, nreal);
+  if (lane < a.n_obs) {
+    a.partial[((long long)lane * a.n_tiles + tile) * kSubs + wave] = mine + held + delta[lane];
+  }
+  if constexpr (HOT)
+    tally_flush(P, lds_tally, a.tally, a.tally_bins);
+}
+
+// ---------------------------------------------------------------------------
 // replay step kernel (FP64): one particle per lane, the reference engine's
 // recorded draws consumed in the reference's order, optional per-step trace
 // ---------------------------------------------------------------------------
@@ -1533,13 +1755,29 @@ int fitting_ppt(StepArgs<R> a, int ppt) {
 template int fitting_ppt<float>(StepArgs<float>, int);
 template int fitting_ppt<double>(StepArgs<double>, int);
 
+// the same for the kernel of one-step launches
+template <typename R, bool POS>
+size_t once_lds(StepArgs<R> &a) {
+  fused_lds<R, 1, POS>(a);
+  a.lds_wave =
+      (int)((once_wave_bytes<R, POS>() + sizeof(double) * (size_t)a.n_obs + 15) & ~size_t(15));
+  return (size_t)a.lds_params + a.lds_hot + (size_t)kSubs * a.lds_wave;
+}
+
 template <typename R, int PPT, bool HOT, bool POS>
 hipError_t launch_fused(StepArgs<R> a, hipStream_t st) {
-  const size_t lds = fused_lds<R, PPT, POS>(a);
-  if (lds > kMaxBulkLds)
-    return hipErrorInvalidValue;
+  size_t lds = fused_lds<R, PPT, POS>(a);
   const void *f = a.max_v == 1 ? (const void *)k_bulk_fused<R, PPT, HOT, POS, 1>
                                : (const void *)k_bulk_fused<R, PPT, HOT, POS, kMaxV>;
+  if constexpr (streams_one_step<R>(PPT)) {
+    if (a.n_steps == 1) {
+      lds = once_lds<R, POS>(a);
+      f = a.max_v == 1 ? (const void *)k_bulk_once<R, PPT, HOT, POS, 1>
+                       : (const void *)k_bulk_once<R, PPT, HOT, POS, kMaxV>;
+    }
+  }
+  if (lds > kMaxBulkLds)
+    return hipErrorInvalidValue;
   if (lds > 64 * 1024) {
     const hipError_t e =
         hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

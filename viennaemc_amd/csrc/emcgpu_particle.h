@@ -30,8 +30,7 @@ struct Math<double> {
   // sin / cos of 2*pi*u, evaluated as the reference does (phi = 2*pi*u)
   static __device__ __forceinline__ void sincos2pi(double u, double *s, double *c) {
     double phi = 2 * 3.14159265358979323846 * u;
-    *s = ::sin(phi);
-    *c = ::cos(phi);
+    ::sincos(phi, s, c);
   }
 };
 
