@@ -1195,30 +1195,42 @@ emcgpu_status get_particles_t(const emcgpu_ctx *c0, int instance, double *k, dou
   const size_t n = in.count;
   if (n == 0)
     return EMCGPU_OK;
-  std::vector<R> hx(n), hy(n), hz(n), he(n), ht(n);
-  std::vector<uint32_t> hv(n);
-  const size_t off = (size_t)in.start;
-  HIPCHK(c, hipMemcpyAsync(hx.data(), (R *)c->kx + off, n * sizeof(R), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(hy.data(), (R *)c->ky + off, n * sizeof(R), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(hz.data(), (R *)c->kz + off, n * sizeof(R), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(he.data(), (R *)c->E + off, n * sizeof(R), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(ht.data(), (R *)c->tau + off, n * sizeof(R), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(hv.data(), c->vs + off, n * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (size_t i = 0; i < n; i++) {
-    if (k) {
-      k[3 * i] = (double)hx[i] / kToNm;
-      k[3 * i + 1] = (double)hy[i] / kToNm;
-      k[3 * i + 2] = (double)hz[i] / kToNm;
-    }
+  // through pinned staging, in pieces where it is smaller than the ensemble
+  const size_t per = 5 * sizeof(R) + sizeof(uint32_t);
+  HIPCHK(c, host_stage(c, n * per));
+  const size_t piece = std::min(n, c->stage_bytes / per);
+  const void *dev[5] = {c->kx, c->ky, c->kz, c->E, c->tau};
+  R *h[5];
+  for (int j = 0; j < 5; j++)
+    h[j] = (R *)c->stage + j * piece;
+  uint32_t *hv = (uint32_t *)(h[4] + piece);
+  for (size_t at = 0; at < n; at += piece) {
+    const size_t m = std::min(piece, n - at), off = (size_t)in.start + at;
+    for (int j = 0; j < 5; j++)
+      HIPCHK(c, hipMemcpyAsync(h[j], (const R *)dev[j] + off, m * sizeof(R), hipMemcpyDeviceToHost,
+                               c->stream));
+    HIPCHK(c, hipMemcpyAsync(hv, c->vs + off, m * sizeof(uint32_t), hipMemcpyDeviceToHost,
+                             c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (k)
+      for (size_t i = 0; i < m; i++) {
+        double *const o = k + 3 * (at + i);
+        o[0] = (double)h[0][i] / kToNm;
+        o[1] = (double)h[1][i] / kToNm;
+        o[2] = (double)h[2][i] / kToNm;
+      }
     if (E)
-      E[i] = (double)he[i];
+      for (size_t i = 0; i < m; i++)
+        E[at + i] = (double)h[3][i];
     if (tau)
-      tau[i] = (double)ht[i] / kToFs;
+      for (size_t i = 0; i < m; i++)
+        tau[at + i] = (double)h[4][i] / kToFs;
     if (valley)
-      valley[i] = (int32_t)(hv[i] >> 16);
+      for (size_t i = 0; i < m; i++)
+        valley[at + i] = (int32_t)(hv[i] >> 16);
     if (sub)
-      sub[i] = (int32_t)(hv[i] & 0xffffu);
+      for (size_t i = 0; i < m; i++)
+        sub[at + i] = (int32_t)(hv[i] & 0xffffu);
   }
   return EMCGPU_OK;
 }
@@ -1247,25 +1259,26 @@ emcgpu_status positions_t(emcgpu_ctx *c, int instance, double *pos, bool get) {
   const size_t n = in.count, off = (size_t)in.start;
   if (n == 0)
     return EMCGPU_OK;
-  std::vector<R> h[3];
   void *dev[3] = {c->px, c->py, c->pz};
-  for (int d = 0; d < 3; d++) {
-    h[d].resize(n);
-    if (!get)
-      for (size_t i = 0; i < n; i++)
-        h[d][i] = (R)(pos[3 * i + d] * 1e9);
+  HIPCHK(c, host_stage(c, n * 3 * sizeof(R)));
+  const size_t piece = std::min(n, c->stage_bytes / (3 * sizeof(R)));
+  R *const h = (R *)c->stage;
+  for (size_t at = 0; at < n; at += piece) {
+    const size_t m = std::min(piece, n - at);
+    for (int d = 0; d < 3; d++) {
+      R *const hd = h + d * piece, *const dd = (R *)dev[d] + off + at;
+      if (!get)
+        for (size_t i = 0; i < m; i++)
+          hd[i] = (R)(pos[3 * (at + i) + d] * 1e9);
+      HIPCHK(c, hipMemcpyAsync(get ? hd : dd, get ? dd : hd, m * sizeof(R),
+                               get ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, c->stream));
+    }
+    HIPCHK(c, hipStreamSynchronize(c->stream));
     if (get)
-      HIPCHK(c, hipMemcpyAsync(h[d].data(), (R *)dev[d] + off, n * sizeof(R),
-                               hipMemcpyDeviceToHost, c->stream));
-    else
-      HIPCHK(c, hipMemcpyAsync((R *)dev[d] + off, h[d].data(), n * sizeof(R),
-                               hipMemcpyHostToDevice, c->stream));
+      for (size_t i = 0; i < m; i++)
+        for (int d = 0; d < 3; d++)
+          pos[3 * (at + i) + d] = (double)h[d * piece + i] * 1e-9;
   }
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (get)
-    for (size_t i = 0; i < n; i++)
-      for (int d = 0; d < 3; d++)
-        pos[3 * i + d] = (double)h[d][i] * 1e-9;
   return EMCGPU_OK;
 }
 
@@ -1379,6 +1392,8 @@ void emcgpu_destroy(emcgpu_ctx *c) {
   dfreet(c->d_partial);
   dfreet(c->d_chunks);
   hfreet(c->h_obs);
+  hfreet(c->stage);
+  dfree(c->work);
   dfreet(c->d_obs0);
   dfree(c->px);
   dfree(c->py);

@@ -2362,8 +2362,9 @@ emcgpu_status emcgpu_deposit(emcgpu_ctx *c, const double *pos, size_t n, double 
   if ((n && !pos) || !grid)
     return fail(c, EMCGPU_ERR_ARG, "pos and grid must be non-NULL");
   DeviceSim &d = *c->dsim;
-  double *dpos = nullptr;
-  HIPCHK(c, hipMalloc((void **)&dpos, std::max<size_t>(n, 1) * 2 * sizeof(double)));
+  Work work;
+  HIPCHK(c, work.get(c, std::max<size_t>(n, 1) * 2 * sizeof(double)));
+  double *dpos = (double *)work.p;
   hipError_t e = hipMemcpy(dpos, pos, n * 2 * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMemcpy(d.d_conc_t, grid, sizeof(double) * d.nn, hipMemcpyHostToDevice);
@@ -2373,7 +2374,6 @@ emcgpu_status emcgpu_deposit(emcgpu_ctx *c, const double *pos, size_t n, double 
     e = hipStreamSynchronize(c->stream);
   if (e == hipSuccess)
     e = hipMemcpy(grid, d.d_conc_t, sizeof(double) * d.nn, hipMemcpyDeviceToHost);
-  (void)hipFree(dpos);
   if (e != hipSuccess)
     return fail(c, EMCGPU_ERR_HIP, "deposit: %s", hipGetErrorString(e));
   return EMCGPU_OK;
@@ -2392,8 +2392,9 @@ emcgpu_status emcgpu_interpolate(emcgpu_ctx *c, const double *ex, const double *
     e2[2 * k] = ex[k];
     e2[2 * k + 1] = ey[k];
   }
-  double *buf = nullptr;
-  HIPCHK(c, hipMalloc((void **)&buf, std::max<size_t>(n, 1) * 4 * sizeof(double)));
+  Work work;
+  HIPCHK(c, work.get(c, std::max<size_t>(n, 1) * 4 * sizeof(double)));
+  double *buf = (double *)work.p;
   double *dpos = buf, *dforce = buf + 2 * std::max<size_t>(n, 1);
   hipError_t e = hipMemcpy(d.d_ex_t, e2.data(), e2.size() * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess)
@@ -2404,7 +2405,6 @@ emcgpu_status emcgpu_interpolate(emcgpu_ctx *c, const double *ex, const double *
     e = hipStreamSynchronize(c->stream);
   if (e == hipSuccess)
     e = hipMemcpy(force, dforce, n * 2 * sizeof(double), hipMemcpyDeviceToHost);
-  (void)hipFree(buf);
   if (e != hipSuccess)
     return fail(c, EMCGPU_ERR_HIP, "interpolate: %s", hipGetErrorString(e));
   return EMCGPU_OK;
@@ -2455,8 +2455,9 @@ emcgpu_status emcgpu_deposit3(emcgpu_ctx *c, const emcgpu_grid3 *g3, const doubl
     return fail(c, EMCGPU_ERR_ARG, "pos and grid must be non-NULL");
   if ((st = pm3_gpu(c)))
     return st;
-  double *buf = nullptr;
-  HIPCHK(c, hipMalloc((void **)&buf, (3 * n + nn) * sizeof(double)));
+  Work work;
+  HIPCHK(c, work.get(c, (3 * n + nn) * sizeof(double)));
+  double *buf = (double *)work.p;
   double *dpos = buf, *dgrid = buf + 3 * n;
   hipError_t e = hipMemcpy(dpos, pos, 3 * n * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess)
@@ -2467,7 +2468,6 @@ emcgpu_status emcgpu_deposit3(emcgpu_ctx *c, const emcgpu_grid3 *g3, const doubl
     e = hipStreamSynchronize(c->stream);
   if (e == hipSuccess)
     e = hipMemcpy(grid, dgrid, nn * sizeof(double), hipMemcpyDeviceToHost);
-  (void)hipFree(buf);
   if (e != hipSuccess)
     return fail(c, EMCGPU_ERR_HIP, "deposit3: %s", hipGetErrorString(e));
   return EMCGPU_OK;
@@ -2485,8 +2485,9 @@ emcgpu_status emcgpu_interpolate3(emcgpu_ctx *c, const emcgpu_grid3 *g3, const d
     return fail(c, EMCGPU_ERR_ARG, "ex, ey, ez, pos and force must be non-NULL");
   if ((st = pm3_gpu(c)))
     return st;
-  double *buf = nullptr;
-  HIPCHK(c, hipMalloc((void **)&buf, (3 * nn + 6 * n) * sizeof(double)));
+  Work work;
+  HIPCHK(c, work.get(c, (3 * nn + 6 * n) * sizeof(double)));
+  double *buf = (double *)work.p;
   double *de = buf, *dpos = buf + 3 * nn, *dforce = dpos + 3 * n;
   hipError_t e = hipMemcpy(de, ex, nn * sizeof(double), hipMemcpyHostToDevice);
   if (e == hipSuccess)
@@ -2502,7 +2503,6 @@ emcgpu_status emcgpu_interpolate3(emcgpu_ctx *c, const emcgpu_grid3 *g3, const d
     e = hipStreamSynchronize(c->stream);
   if (e == hipSuccess)
     e = hipMemcpy(force, dforce, 3 * n * sizeof(double), hipMemcpyDeviceToHost);
-  (void)hipFree(buf);
   if (e != hipSuccess)
     return fail(c, EMCGPU_ERR_HIP, "interpolate3: %s", hipGetErrorString(e));
   return EMCGPU_OK;
@@ -2536,8 +2536,9 @@ emcgpu_status emcgpu_efield3(emcgpu_ctx *c, const emcgpu_grid3 *g3, double vt,
     }
   if ((st = pm3_gpu(c)))
     return st;
-  double *buf = nullptr;
-  HIPCHK(c, hipMalloc((void **)&buf, 4 * nn * sizeof(double) + 3 * nn));
+  Work work;
+  HIPCHK(c, work.get(c, 4 * nn * sizeof(double) + 3 * nn));
+  double *buf = (double *)work.p;
   double *dpot = buf, *de = buf + nn;
   signed char *dbc = (signed char *)(buf + 4 * nn);
   hipError_t e = hipMemcpy(dpot, pot, nn * sizeof(double), hipMemcpyHostToDevice);
@@ -2552,7 +2553,6 @@ emcgpu_status emcgpu_efield3(emcgpu_ctx *c, const emcgpu_grid3 *g3, double vt,
   double *outs[3] = {ex, ey, ez};
   for (int d = 0; d < 3 && e == hipSuccess; d++)
     e = hipMemcpy(outs[d], de + d * nn, nn * sizeof(double), hipMemcpyDeviceToHost);
-  (void)hipFree(buf);
   if (e != hipSuccess)
     return fail(c, EMCGPU_ERR_HIP, "efield3: %s", hipGetErrorString(e));
   return EMCGPU_OK;

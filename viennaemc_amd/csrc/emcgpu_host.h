@@ -109,6 +109,12 @@ struct emcgpu_ctx {
   // memory that the reduction kernels write: a read waits for the stream and
   // copies nothing from the device
   double *h_obs = nullptr;
+  // of the calls on host arrays, kept up to kKeepBytes each and freed with the
+  // context: device workspace, pinned staging of particle transfers
+  void *work = nullptr;
+  size_t work_bytes = 0;
+  unsigned char *stage = nullptr;
+  size_t stage_bytes = 0;
   size_t obs_bytes = 0;
   int obs_steps = 0;
   // timing
@@ -200,6 +206,49 @@ void hfreet(T *&p) {
     (void)hipHostFree(p);
     p = nullptr;
   }
+}
+
+// workspaces of calls on host arrays that a context keeps
+constexpr size_t kKeepBytes = size_t(64) << 20;
+
+// `bytes` of device memory for the duration of a call: the context's
+// workspace, or memory of its own where more is needed than is kept
+struct Work {
+  void *p = nullptr;
+  bool own = false;
+  ~Work() {
+    if (own)
+      (void)hipFree(p);
+  }
+  hipError_t get(emcgpu_ctx *c, size_t bytes) {
+    if (bytes > kKeepBytes) {
+      own = true;
+      return hipMalloc(&p, bytes);
+    }
+    if (bytes > c->work_bytes) {
+      dfree(c->work);
+      c->work_bytes = 0;
+      const hipError_t e = hipMalloc(&c->work, bytes);
+      if (e != hipSuccess)
+        return e;
+      c->work_bytes = bytes;
+    }
+    p = c->work;
+    return hipSuccess;
+  }
+};
+
+// pinned staging of at least min(bytes, kKeepBytes), nothing pending on it
+inline hipError_t host_stage(emcgpu_ctx *c, size_t bytes) {
+  bytes = bytes < kKeepBytes ? bytes : kKeepBytes;
+  if (bytes <= c->stage_bytes)
+    return hipSuccess;
+  hfreet(c->stage);
+  c->stage_bytes = 0;
+  const hipError_t e = hipHostMalloc((void **)&c->stage, bytes, hipHostMallocDefault);
+  if (e == hipSuccess)
+    c->stage_bytes = bytes;
+  return e;
 }
 
 inline emcgpu_status check_instance(emcgpu_ctx *c, int instance) {
