@@ -359,6 +359,13 @@ struct DimTab {
   float wl, wr;           // restriction: weights of fine nodes f-1, f+1 (mirror folded)
 };
 
+// where the Poisson workgroup keeps its multigrid data: all in LDS (up to
+// about 11k nodes); the fine grid's residual, which a V-cycle writes and reads
+// once, in the global workspace and the rest in LDS (up to about 15k); all in
+// the workspace.  Equilibrium of the 126 x 101 MOSFET grid, 32 V-cycles, with
+// the call: 6.82 ms all in the workspace, 4.96 ms with the residual alone.
+constexpr int kMgLds = 0, kMgResGlobal = 1, kMgGlobal = 2;
+
 // Poisson + E-field on one workgroup
 template <typename R>
 struct DevFieldArgs {
@@ -401,8 +408,8 @@ struct DevFieldArgs {
   // dynamic LDS layout (float offsets; tab and cmask in bytes)
   int lds_res, lds_rc, lds_sc, lds_tab, lds_cmask;
   int lds_dummy;  // float offset of one scratch word per thread
-  // the same layout in global memory (L2-resident) when it exceeds the
-  // LDS, null when it fits
+  // global memory (L2-resident) of what does not fit: the fine grid's
+  // residual (kMgResGlobal) or the whole layout (kMgGlobal)
   float *mg_ws;
   // fine-grid thread map: a thread owns column (tid mod 2^cw_log2) of a row
   // block; half-row map (red-black sweeps, node pairs) and full-row map,

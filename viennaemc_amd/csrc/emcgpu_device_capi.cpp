@@ -22,7 +22,7 @@
 
 namespace emcgpu {
 template <typename R>
-hipError_t dev_launch_field(const DevFieldArgs<R> *args_dev, size_t lds, bool ws, hipStream_t st);
+hipError_t dev_launch_field(const DevFieldArgs<R> *args_dev, size_t lds, int ws, hipStream_t st);
 template <typename R>
 hipError_t dev_launch_efield(const DevFieldArgs<R> *args_dev, int nn, hipStream_t st);
 template <typename R>
@@ -110,7 +110,7 @@ struct DeviceSim {
   std::vector<DimTab> tab;
   std::vector<uint8_t> lmask;
   size_t mg_lds = 0;
-  bool mg_global = false;  // the multigrid data exceed the LDS: global workspace d_mg_ws
+  int mg_place = kMgLds;  // where the multigrid data live (kMg*), beyond the LDS in d_mg_ws
   int mg_nodes = 0;  // nodes of all levels
   int lds_res = 0, lds_rc = 0, lds_sc = 0, lds_tab = 0, lds_cmask = 0, wave_level = 0;
   int lds_dummy = 0;
@@ -667,15 +667,25 @@ emcgpu_status build_multigrid(emcgpu_ctx *c, DeviceSim &d) {
   }
   d.mg_nodes = off;
   const int n0 = d.lev[0].nx * d.lev[0].ny, nc = off - n0;
-  d.lds_res = off;
-  d.lds_rc = d.lds_res + n0;
-  d.lds_sc = d.lds_rc + nc;
-  d.lds_tab = (int)(((size_t)(d.lds_sc + nc) * sizeof(float) + 15) & ~(size_t)15);
-  d.lds_cmask = d.lds_tab + (int)(d.tab.size() * sizeof(DimTab));
-  d.mg_lds = ((size_t)d.lds_cmask + nc + 15) & ~(size_t)15;
-  // one word per thread for the fine-grid passes' off-grid slots
-  d.lds_dummy = (int)(d.mg_lds / sizeof(float));
-  d.mg_lds += kDevThreads * sizeof(float);
+  // corrections of every level, residual, coarse right-hand sides and shifts,
+  // transfer tables, masks, one word per thread for the fine-grid passes'
+  // off-grid slots; with the fine grid's residual in global memory the LDS
+  // holds the next level's
+  const int n1 = nl > 1 ? d.lev[1].nx * d.lev[1].ny : 0;
+  auto layout = [&](int n_res) {
+    d.lds_res = off;
+    d.lds_rc = d.lds_res + n_res;
+    d.lds_sc = d.lds_rc + nc;
+    d.lds_tab = (int)(((size_t)(d.lds_sc + nc) * sizeof(float) + 15) & ~(size_t)15);
+    d.lds_cmask = d.lds_tab + (int)(d.tab.size() * sizeof(DimTab));
+    d.mg_lds = ((size_t)d.lds_cmask + nc + 15) & ~(size_t)15;
+    d.lds_dummy = (int)(d.mg_lds / sizeof(float));
+    d.mg_lds += kDevThreads * sizeof(float);
+    return d.mg_lds <= (size_t)kDevMaxLds;
+  };
+  d.mg_place = layout(n0) ? kMgLds : layout(n1) ? kMgResGlobal : kMgGlobal;
+  if (d.mg_place == kMgGlobal)
+    layout(n0);
   d.wave_level = nl;
   for (int l = 1; l < nl; l++)
     if (d.lev[l].nx * d.lev[l].ny <= 256) {
@@ -774,9 +784,6 @@ emcgpu_status build_multigrid(emcgpu_ctx *c, DeviceSim &d) {
   const int rh = kDevThreads >> d.hcw_log2, rf = kDevThreads >> d.fcw_log2;
   d.nph = (d.ext[1] + rh - 1) / rh;
   d.npf = (d.ext[1] + rf - 1) / rf;
-  // levels beyond the LDS: the same layout in a global workspace (the
-  // workgroup then reads them through L2)
-  d.mg_global = d.mg_lds > (size_t)kDevMaxLds;
   // the Poisson passes' index maths (idiv) is exact below 2^22 nodes
   if ((size_t)d.mg_nodes + d.mg_lds / sizeof(float) >= ((size_t)1 << 22))
     return fail(c, EMCGPU_ERR_ARG, "a %d x %d grid exceeds the Poisson solver (%d nodes)",
@@ -862,7 +869,9 @@ emcgpu_status upload_device(emcgpu_ctx *c, DeviceSim &d) {
   ST(dalloc(c, d.d_q64, np));
   ST(dalloc(c, d.d_s64, np));
   ST(dalloc(c, d.d_rs0, np));
-  if (d.mg_global)
+  if (d.mg_place == kMgResGlobal)
+    ST(dalloc(c, d.d_mg_ws, nn));
+  if (d.mg_place == kMgGlobal)
     ST(dalloc(c, d.d_mg_ws, (d.mg_lds + sizeof(float) - 1) / sizeof(float)));
   {
     std::vector<float> w(np, 0.0f), hw(np, 0.0f);
@@ -1134,7 +1143,7 @@ DevFieldArgs<R> field_args(const emcgpu_ctx *c, const DeviceSim &d) {
   a.lds_tab = d.lds_tab;
   a.lds_cmask = d.lds_cmask;
   a.lds_dummy = d.lds_dummy;
-  a.mg_ws = d.mg_global ? d.d_mg_ws : nullptr;
+  a.mg_ws = d.mg_place == kMgLds ? nullptr : d.d_mg_ws;
   a.hcw_log2 = d.hcw_log2;
   a.nph = d.nph;
   a.fcw_log2 = d.fcw_log2;
@@ -1299,7 +1308,7 @@ emcgpu_status put_fargs(emcgpu_ctx *c, DeviceSim &d, int slot, const DevFieldArg
 template <typename R>
 emcgpu_status run_field(emcgpu_ctx *c, DeviceSim &d, DevFieldArgs<R> a) {
   ST(put_fargs<R>(c, d, 2, a));
-  HIPCHK(c, dev_launch_field<R>(fargs_slot<R>(d, 2), d.mg_lds, d.mg_global, c->stream));
+  HIPCHK(c, dev_launch_field<R>(fargs_slot<R>(d, 2), d.mg_lds, d.mg_place, c->stream));
   return EMCGPU_OK;
 }
 
@@ -1714,7 +1723,7 @@ emcgpu_status launch_step(emcgpu_ctx *c, DeviceSim &d, bool reset_bc) {
     }
     HIPCHK(c, dev_launch_green(ga, green_iters(d), d.green_blocks, c->stream));
   }
-  HIPCHK(c, dev_launch_field<R>(fargs_slot<R>(d, reset_bc ? 1 : 0), d.mg_lds, d.mg_global,
+  HIPCHK(c, dev_launch_field<R>(fargs_slot<R>(d, reset_bc ? 1 : 0), d.mg_lds, d.mg_place,
                                  c->stream));
   if (split_efield(d) && !corr)
     HIPCHK(c, dev_launch_efield<R>(fargs_slot<R>(d, reset_bc ? 1 : 0), (int)d.nn, c->stream));

@@ -1275,10 +1275,10 @@ __device__ __forceinline__ void mg_sweep_c(const DevFieldArgs<R> &a, const MGSha
 // folded in) of a fine-level field src (level l, dense nx * ny) into the
 // coarse level l+1 array dst; masked coarse nodes get 0; zero_d clears the
 // coarse correction
-template <typename R, typename T>
+template <typename R, typename T, typename Src>
 __device__ __forceinline__ void mg_restrict_to(const DevFieldArgs<R> &a, const MGShared &m, int l,
-                                               const float *src, float *dst, bool zero_d,
-                                               T team, bool keep_masked = false) {
+                                               Src src, float *dst, bool zero_d, T team,
+                                               bool keep_masked = false) {
   const MGLevel L = a.lev[l], C = a.lev[l + 1];
   const uint8_t *cmask = m.cmask + (C.off - m.n0);
   const DimTab *CX = m.tab + C.tx, *CY = m.tab + C.ty;
@@ -1527,8 +1527,18 @@ __device__ __forceinline__ void mg_direct(const DevFieldArgs<R> &a, const MGShar
   __syncthreads();
 }
 
+// the level-0 residual of the Poisson kernel's memory variants: beside the
+// corrections, or (kMgResGlobal) in the global workspace
+template <int MG, typename R>
+__device__ __forceinline__ auto mg_res0(const DevFieldArgs<R> &a, const MGShared &m) {
+  if constexpr (MG == kMgResGlobal)
+    return glb(a.mg_ws);
+  else
+    return m.res;
+}
+
 // z = V-cycle(r) into m.d[0 .. n0)
-template <typename R>
+template <int MG, typename R>
 __device__ __forceinline__ void mg_vcycle(const DevFieldArgs<R> &a, const MGShared &m) {
   const int nl = a.n_levels;
   for (int k = threadIdx.x; k < a.nn; k += kDevThreads)
@@ -1562,12 +1572,18 @@ __device__ __forceinline__ void mg_vcycle(const DevFieldArgs<R> &a, const MGShar
         const float rk =
             v[u].x - ((diag + v[u].y) * m.d[f[u].k] -
                       (hfx * (m.d[f[u].il] + m.d[f[u].ir]) + hfy * (m.d[f[u].jd] + m.d[f[u].ju])));
-        // m.res[k] (m.res = m.d + lds_res), the scratch word off the grid
-        m.d[f[u].ok ? a.lds_res + f[u].k : f[u].k] = v[u].y >= kBigShift ? 0.0f : rk;
+        const float rm = v[u].y >= kBigShift ? 0.0f : rk;
+        if constexpr (MG == kMgResGlobal) {
+          if (f[u].ok)
+            mg_res0<MG>(a, m)[f[u].k] = rm;
+        } else {
+          // m.res[k] (m.res = m.d + lds_res), the scratch word off the grid
+          m.d[f[u].ok ? a.lds_res + f[u].k : f[u].k] = rm;
+        }
       }
     }
     __syncthreads();
-    mg_restrict_to(a, m, 0, m.res, m.rc + (a.lev[1].off - m.n0), true, BlockTeam());
+    mg_restrict_to(a, m, 0, mg_res0<MG>(a, m), m.rc + (a.lev[1].off - m.n0), true, BlockTeam());
   }
   // the coarse level below which the hierarchy is replaced by its exact
   // inverse (when the Jacobian shift is negligible there), or handed to one
@@ -1610,17 +1626,18 @@ __device__ __forceinline__ void mg_vcycle(const DevFieldArgs<R> &a, const MGShar
 
 // diagonal shifts of the coarse levels from the level-0 one (lumped
 // Galerkin P^T diag(sigma) P)
-template <typename R>
+template <int MG, typename R>
 __device__ __forceinline__ void mg_shift_down(const DevFieldArgs<R> &a, const MGShared &m) {
   const int nl = a.n_levels;
   if (nl == 1)
     return;
+  const auto res0 = mg_res0<MG>(a, m);
   for (int k = threadIdx.x; k < a.nn; k += kDevThreads) {
     const float sk = a.rs0[k].y;
-    m.res[k] = sk >= kBigShift ? 0.0f : sk;
+    res0[k] = sk >= kBigShift ? 0.0f : sk;
   }
   __syncthreads();
-  mg_restrict_to(a, m, 0, m.res, m.sc + (a.lev[1].off - m.n0), false, BlockTeam(), true);
+  mg_restrict_to(a, m, 0, res0, m.sc + (a.lev[1].off - m.n0), false, BlockTeam(), true);
   for (int l = 1; l < nl - 1; ++l) {
     // the restriction input: the finer level's shift without its Dirichlet
     // values
@@ -1643,13 +1660,12 @@ __device__ __forceinline__ void mg_shift_down(const DevFieldArgs<R> &a, const MG
 // vectors and the update are FP64; the CG preconditioner is one FP32
 // multigrid V-cycle.  Then calcEField (PMSchemes/emcEFieldCalculation.hpp:
 // 13-81).
-template <typename R, bool WS>
+// MG: where the multigrid data live (kMg*)
+template <typename R, int MG>
 __global__ __launch_bounds__(kDevThreads) void k_dev_field(const DevFieldArgs<R> *__restrict__ args) {
   const DevFieldArgs<R> &a = *args;
   extern __shared__ __align__(16) float lds[];
-  // the multigrid data: in LDS, or with WS (grids whose levels exceed the
-  // LDS) in a global workspace of the same layout, kept in L2
-  float *const mg = WS ? a.mg_ws : lds;
+  float *const mg = MG == kMgGlobal ? a.mg_ws : lds;
   __shared__ double red[kDevThreads / 64];
   const int tid = threadIdx.x;
   const int nx = a.nx, ny = a.ny, nn = a.nn;
@@ -1791,7 +1807,7 @@ __global__ __launch_bounds__(kDevThreads) void k_dev_field(const DevFieldArgs<R>
       if (fm <= a.tol * scale || it >= a.max_iter || vcycles >= a.max_vcycles)
         break;
       if (a.equilibrium || it == 0)
-        mg_shift_down(a, m);
+        mg_shift_down<MG>(a, m);
       // conjugate gradients on A x = F (A = -Jacobian, symmetric in the
       // control-volume inner product), x0 = 0
       // inexact Newton away from the root: the FP32-preconditioned CG
@@ -1808,7 +1824,7 @@ __global__ __launch_bounds__(kDevThreads) void k_dev_field(const DevFieldArgs<R>
         p64[k] = 0.0;
       }
       for (int pit = 0; pit < a.max_pcg; ++pit) {
-        mg_vcycle(a, m);  // z = M^-1 r in m.d[0 .. nn)
+        mg_vcycle<MG>(a, m);  // z = M^-1 r in m.d[0 .. nn)
         ++vcycles;
         double rz = 0.0;
         for (int k0 = tid; k0 < np; k0 += kPad) {
@@ -1977,23 +1993,24 @@ hipError_t dev_launch_efield(const DevFieldArgs<R> *args_dev, int nn, hipStream_
 // the caller): dynamic indexing of the level table would otherwise copy the
 // whole block to scratch
 template <typename R>
-hipError_t dev_launch_field(const DevFieldArgs<R> *args_dev, size_t lds, bool ws, hipStream_t st) {
-  if (ws) {  // the multigrid data in the global workspace (args_dev->mg_ws)
-    hipLaunchKernelGGL((k_dev_field<R, true>), dim3(1), dim3(kDevThreads), 0, st, args_dev);
+hipError_t dev_launch_field(const DevFieldArgs<R> *args_dev, size_t lds, int mg, hipStream_t st) {
+  if (mg == kMgGlobal) {  // the multigrid data in the global workspace (args_dev->mg_ws)
+    hipLaunchKernelGGL((k_dev_field<R, kMgGlobal>), dim3(1), dim3(kDevThreads), 0, st, args_dev);
     return hipGetLastError();
   }
   if (lds > (size_t)kDevMaxLds)
     return hipErrorInvalidValue;
+  const void *f = mg == kMgResGlobal ? (const void *)k_dev_field<R, kMgResGlobal>
+                                     : (const void *)k_dev_field<R, kMgLds>;
   if (lds > 65536) {
-    hipError_t e = hipFuncSetAttribute((const void *)k_dev_field<R, false>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) {
       (void)hipGetLastError();
       return e;
     }
   }
-  hipLaunchKernelGGL((k_dev_field<R, false>), dim3(1), dim3(kDevThreads), lds, st, args_dev);
-  return hipGetLastError();
+  void *args[] = {(void *)&args_dev};
+  return hipLaunchKernel(f, dim3(1), dim3(kDevThreads), args, lds, st);
 }
 
 // the step kernel with an FP64 or an R deposit grid in LDS
@@ -2510,7 +2527,7 @@ hipError_t dev_launch_green_expand(const double *Ainv, long long lda, const int 
 }
 
 #define EMCGPU_DEV_INST(R)                                                                   \
-  template hipError_t dev_launch_field<R>(const DevFieldArgs<R> *, size_t, bool, hipStream_t);      \
+  template hipError_t dev_launch_field<R>(const DevFieldArgs<R> *, size_t, int, hipStream_t);      \
   template hipError_t dev_launch_efield<R>(const DevFieldArgs<R> *, int, hipStream_t);        \
   template hipError_t dev_launch_step<R>(const DevStepArgs<R> &, const DevContactArgs<R> &, int, \
                                          int, size_t, hipStream_t);                           \
