@@ -570,9 +570,17 @@ __device__ __forceinline__ void dev_reduce_rows(const DevContactArgs<R> &a, int 
     return;
   const int b0 = chunk * a.rows_per_chunk;
   const int b1 = b0 + a.rows_per_chunk < a.n_blocks_dep ? b0 + a.rows_per_chunk : a.n_blocks_dep;
+  // the rows in order, sixteen loads in flight at a time
   double s = 0.0;
-  for (int b = b0; b < b1; ++b)
-    s += (double)a.dep[(long long)b * nn + k];
+  for (int b = b0; b < b1; b += 16) {
+    R v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      v[u] = b + u < b1 ? a.dep[(long long)(b + u) * nn + k] : R(0);
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      s += (double)v[u];
+  }
   a.dpart[(long long)chunk * nn + k] = s;
   if (a.n_blocks_dep == 1)  // the atomic deposit accumulates in row 0
     a.dep[k] = R(0);
@@ -601,9 +609,35 @@ __global__ __launch_bounds__(kDevStepThreads) void k_dev_rank_rows(DevStepArgs<R
 // ohmic contacts: per node, array-order offsets of the segments' particles,
 // then keep while nrPart < expected, inject ceil(expected - kept)
 // ---------------------------------------------------------------------------
+// inclusive sum over the threads of a 256-thread block up to this one; *total
+// gets the block's (one barrier: wave scans, then the waves before)
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t *total) {
+  __shared__ uint32_t ws[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t o = __shfl_up(v, d, 64);
+    v += lane >= d ? o : 0u;
+  }
+  if (lane == 63)
+    ws[wave] = v;
+  __syncthreads();
+  uint32_t all = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    v += w < wave ? ws[w] : 0u;
+    all += ws[w];
+  }
+  *total = all;
+  return v;
+}
+
+// bound by latency: the counts are loaded once, sixteen per thread (4096
+// segments on 256 CUs), and scanned across the block with one barrier: 8.8 ->
+// 6.6 us on a 200 x 50 resistor of 2 M particles, 8.9 -> 6.2 us on a gated
+// device of 60 k (the sixteen passes over memory with four barriers each)
 template <typename R>
 __global__ __launch_bounds__(256) void k_dev_contact_scan(DevContactArgs<R> a) {
-  __shared__ uint32_t sc[256];
   const int slot = blockIdx.x, tid = threadIdx.x;
   const int S = a.n_segments;
   const uint32_t *cnt = a.seg_cnt + (long long)slot * S;  // row of the [slot][segment] counts
@@ -611,42 +645,32 @@ __global__ __launch_bounds__(256) void k_dev_contact_scan(DevContactArgs<R> a) {
   const int per = (S + 255) / 256;
   const int b0 = tid * per < S ? tid * per : S;
   const int b1 = b0 + per < S ? b0 + per : S;
-  // the thread's counts, sixteen loads in flight at a time
+  uint32_t v[16];
+#pragma unroll
+  for (int u = 0; u < 16; ++u)
+    v[u] = b0 + u < b1 ? cnt[b0 + u] : 0u;
   uint32_t tot = 0;
-  for (int b = b0; b < b1; b += 16) {
-    uint32_t v[16];
 #pragma unroll
-    for (int u = 0; u < 16; ++u)
-      v[u] = b + u < b1 ? cnt[b + u] : 0u;
+  for (int u = 0; u < 16; ++u)
+    tot += v[u];
+  for (int b = b0 + 16; b < b1; ++b)
+    tot += cnt[b];
+  uint32_t all;
+  uint32_t run = block_scan(tot, &all) - tot;
 #pragma unroll
-    for (int u = 0; u < 16; ++u)
-      tot += v[u];
+  for (int u = 0; u < 16; ++u) {
+    if (b0 + u < b1)
+      off[b0 + u] = run;
+    run += v[u];
   }
-  sc[tid] = tot;
-  __syncthreads();
-  for (int d = 1; d < 256; d <<= 1) {
-    const uint32_t t = tid >= d ? sc[tid - d] : 0u;
-    __syncthreads();
-    sc[tid] += t;
-    __syncthreads();
-  }
-  uint32_t run = sc[tid] - tot;
-  for (int b = b0; b < b1; b += 16) {
-    uint32_t v[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u)
-      v[u] = b + u < b1 ? cnt[b + u] : 0u;
-#pragma unroll
-    for (int u = 0; u < 16; ++u)
-      if (b + u < b1) {
-        off[b + u] = run;
-        run += v[u];
-      }
+  for (int b = b0 + 16; b < b1; ++b) {
+    off[b] = run;
+    run += cnt[b];
   }
   // the node's counts (no atomics: the resolve kernel totals them per
   // contact)
   if (tid == 0) {
-    const long long total = sc[255];
+    const long long total = all;
     const double e = a.slot_exp[slot];
     const long long ce = (long long)ceil(e);
     const long long kept = total < ce ? total : ce;
@@ -695,7 +719,6 @@ __global__ __launch_bounds__(256) void k_dev_resolve(DevContactArgs<R> a) {
   const long long bi = (long long)blockIdx.x - nA;
   const long long t = bi * 256 + tid;
   {  // prefix of the injections over the ohmic nodes (4 nodes per thread)
-    __shared__ int ws[256];
     int v[4], run = 0;
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -703,15 +726,8 @@ __global__ __launch_bounds__(256) void k_dev_resolve(DevContactArgs<R> a) {
       v[u] = q < a.n_slots ? a.slot_inj[q] : 0;
       run += v[u];
     }
-    ws[tid] = run;
-    __syncthreads();
-    for (int d = 1; d < 256; d <<= 1) {
-      const int o = tid >= d ? ws[tid - d] : 0;
-      __syncthreads();
-      ws[tid] += o;
-      __syncthreads();
-    }
-    int acc = ws[tid] - run;
+    uint32_t all;
+    int acc = (int)block_scan((uint32_t)run, &all) - run;
     if (tid == 0)
       pre[0] = 0;
 #pragma unroll
@@ -799,10 +815,19 @@ __global__ __launch_bounds__(256) void k_dev_reduce(DevContactArgs<R> a, int com
   const int k = blockIdx.x * 256 + threadIdx.x;
   const int nn = a.g.nn;
   if (k < nn) {
+    // the chunks in order, sixteen loads in flight at a time
     double s = 0.0;
-    for (int c = 0; c < a.n_chunks; ++c)
-      s += a.dpart[(long long)c * nn + k];
-    s += a.corr[k];
+    const double corr = a.corr[k];
+    for (int c = 0; c < a.n_chunks; c += 16) {
+      double v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        v[u] = c + u < a.n_chunks ? a.dpart[(long long)(c + u) * nn + k] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        s += v[u];
+    }
+    s += corr;
     a.corr[k] = 0.0;
     a.nrpart[k] = s;
     const double cn = s * a.cfac[k];
