@@ -666,11 +666,12 @@ emcgpu_status upload_params(emcgpu_ctx *c, double dt_s) {
 // 2.6 / 3.0 / 3.8, 150k 3.2 / 3.3 / 4.0, 200k 3.6 / 3.4 / 4.0, 300k 4.2 / 3.9
 // / 4.3, 400k 5.7 / 4.4 / 4.3, 1M 10.6 / 7.5 / 5.8; FP64 10k 3.4 / 4.4 / 5.7,
 // 150k 5.7 / 5.6 / 5.8, 300k 9.0 / 7.3 / 7.4, 400k 11.7 / 9.6 / 7.6, 1M 24.2 /
-// 17.2 / 12.9.  One-step launches in FP64 stream their particles and take
-// eight per lane (screened cooling, 1M: 51.7 us with four, 41.8 with eight).
+// 17.2 / 12.9.  One-step launches in FP64 of models with one valley stream
+// their particles and take eight per lane (screened cooling, 1M: 51.7 us with
+// four, 41.8 with eight).
 int default_ppt(const emcgpu_ctx *c, bool one_step) {
   constexpr long long kFill = 1280 * 64;
-  if (one_step && c->precision == EMCGPU_FP64 && c->capacity >= 8 * kFill)
+  if (one_step && c->max_v == 1 && c->precision == EMCGPU_FP64 && c->capacity >= 8 * kFill)
     return 8;
   return c->capacity >= 4 * kFill ? 4 : c->capacity >= 2 * kFill ? 2 : 1;
 }

@@ -622,7 +622,12 @@ __global__ __launch_bounds__(kTile, PPT == 1 ? 1 : sizeof(R) == 8 ? 3 : 6) void 
 // with 0.13 events per particle and step, 1M: 53.6 -> 41.8 us per step with
 // 8 per lane, 4M: 134.7 -> 106.6), and for small ensembles (50k FP32: 11.9 ->
 // 10.8).  In FP32 the stores of single particles cost more than the passes
-// they save (4M Si: 47.4 us with the particles in LDS, 55.5 streamed).
+// they save (4M Si: 47.4 us with the particles in LDS, 55.5 streamed).  For
+// models of one valley: with more, the passes' and the stream's registers
+// do not fit side by side (FP64, two valleys, 8M: 242 us in LDS with 4 per
+// lane, 318 streamed with 8).  With one particle per lane nothing is queued:
+// the particle stays in its lane and the wave stores whole lines at the end
+// (8M Si, FP32 134 -> 121 us, FP64 385 -> 371 against queueing them).
 // ---------------------------------------------------------------------------
 template <typename R>
 constexpr bool streams_one_step(int ppt) {
@@ -637,10 +642,10 @@ constexpr size_t once_wave_bytes() {
   return (size_t)kOnceQueue * ((POS ? 7 : 4) * sizeof(R) + sizeof(uint32_t) + sizeof(uint16_t));
 }
 
-template <typename R, int PPT, bool HOT, bool POS, int NV>
+template <typename R, int PPT, bool HOT, bool POS>
 __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(StepArgs<R> a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  constexpr int TS = kTile * PPT, Q = kOnceQueue;
+  constexpr int TS = kTile * PPT, Q = kOnceQueue, NV = 1;
   const int tile = blockIdx.x;
   const int inst = tile_instance(a.unit_inst, tile, TS);
   const InstDev<R> *P = stage_params(lds, a.inst + inst, a.lds_params);
@@ -762,15 +767,13 @@ __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(Ste
       if (v != v0 || sub != sub00) {
         atomicAdd(delta + sub0 + v0 * a.max_deg + sub00, -1.0);
         atomicAdd(delta + sub0 + v * a.max_deg + sub, 1.0);
-        if (NV > 1 && v != v0) {
-          atomicAdd(delta + 2 + 3 * v0, -1.0);
-          atomicAdd(delta + 2 + 3 * v, 1.0);
-        }
       }
       if (busy && (!(rem > R(0)) || ev >= kMaxEventsPerStep)) {
-        const long long gi = store(idx, kx, ky, kz, E, tau - dt, pos);
-        a.vs[gi] = ((uint32_t)v << 16) | (uint32_t)sub;
-        sums.add(P, kane(v), v, sub, kx, ky, kz, E);
+        if constexpr (PPT > 1) {
+          const long long gi = store(idx, kx, ky, kz, E, tau - dt, pos);
+          a.vs[gi] = ((uint32_t)v << 16) | (uint32_t)sub;
+          sums.add(P, kane(v), v, sub, kx, ky, kz, E);
+        }
         busy = false;
       }
     }
@@ -783,25 +786,48 @@ __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(Ste
     Part p = next;
     load(j + 1, next);
     const int vv = (int)(p.vs >> 16), ss = (int)(p.vs & 0xffffu);
-    for (int k = 0; k < a.max_v; ++k) {
-      int n = 0;
-      for (int d = 0; d < a.max_deg; ++d) {
-        const int c = (int)__popcll(__ballot(p.valid && (NV == 1 || vv == k) && ss == d));
-        n += c;
-        held += (lane == sub0 + k * a.max_deg + d) ? (double)c : 0.0;
-      }
-      held += (lane == 2 + 3 * k) ? (double)n : 0.0;
+    int n = 0;
+    for (int d = 0; d < a.max_deg; ++d) {
+      const int c = (int)__popcll(__ballot(p.valid && ss == d));
+      n += c;
+      held += (lane == sub0 + d) ? (double)c : 0.0;
     }
+    held += (lane == 2) ? (double)n : 0.0;
     bool pend = false;
+    R en = R(0);
     if (p.valid) {
-      R en = R(0);
-      drift<R, POS>(P, kane(vv), (dt < p.tau) ? dt : p.tau, p.x, p.y, p.z, en, NV == 1 ? 0 : vv, ss,
-                    p.pos);
+      drift<R, POS>(P, kane(vv), (dt < p.tau) ? dt : p.tau, p.x, p.y, p.z, en, 0, ss, p.pos);
       pend = dt - p.tau > R(0);
-      if (!pend) {
+      if (PPT > 1 && !pend) {
         store(j * 64 + lane, p.x, p.y, p.z, en, p.tau - dt, p.pos);
         sums.add(P, kane(vv), vv, ss, p.x, p.y, p.z, en);
       }
+    }
+    if constexpr (PPT == 1) {
+      // one particle per lane: it stays there, and all of a wave's leave at once
+      kx = p.x;
+      ky = p.y;
+      kz = p.z;
+      tau = p.tau;
+      v = vv;
+      sub = ss;
+      idx = lane;
+      if constexpr (POS) {
+        pos[0] = p.pos[0];
+        pos[1] = p.pos[1];
+        pos[2] = p.pos[2];
+      }
+      E = pend ? energy_of(kane(v), kx, ky, kz) : en;
+      rem = dt - tau;
+      busy = pend;
+      passes(1);
+      if (p.valid) {
+        const long long gi = store(lane, kx, ky, kz, E, tau - dt, pos);
+        if (pend)
+          a.vs[gi] = ((uint32_t)v << 16) | (uint32_t)sub;
+        sums.add(P, kane(v), v, sub, kx, ky, kz, E);
+      }
+      break;
     }
     const unsigned long long m = __ballot(pend);
     if (pend) {
@@ -1783,10 +1809,9 @@ hipError_t launch_fused(StepArgs<R> a, hipStream_t st) {
   const void *f = a.max_v == 1 ? (const void *)k_bulk_fused<R, PPT, HOT, POS, 1>
                                : (const void *)k_bulk_fused<R, PPT, HOT, POS, kMaxV>;
   if constexpr (streams_one_step<R>(PPT)) {
-    if (a.n_steps == 1) {
+    if (a.n_steps == 1 && a.max_v == 1) {
       lds = once_lds<R, POS>(a);
-      f = a.max_v == 1 ? (const void *)k_bulk_once<R, PPT, HOT, POS, 1>
-                       : (const void *)k_bulk_once<R, PPT, HOT, POS, kMaxV>;
+      f = (const void *)k_bulk_once<R, PPT, HOT, POS>;
     }
   }
   if (lds > kMaxBulkLds)
