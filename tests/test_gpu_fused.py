@@ -84,3 +84,89 @@ def test_one_step_launches(model, dt, ppl):
     in one to eight chunks of 64, the last one ragged, with few and with
     mostly scattering particles"""
     _run(MODELS[model], 1801, 12, dt, ppl, 1)
+
+
+# dt such that about 4 % and most of the particles scatter in a step
+RARE, MANY = {"si_jacoboni": 0.2e-15, "two_valley": 1e-15}, 12e-15
+
+
+@pytest.mark.parametrize("spl", [1, 3, 4, 5])
+@pytest.mark.parametrize("n", [1, 65, 1801])
+@pytest.mark.parametrize("model", ["si_jacoboni", "two_valley"])
+def test_short_launches_one_per_lane(model, n, spl):
+    """one particle per lane: in registers up to four steps per launch, in LDS
+    from five on"""
+    _run(MODELS[model], n, 10, MANY, 1, spl)
+
+
+@pytest.mark.parametrize("ppl", [1, 2, 4, 8])
+@pytest.mark.parametrize("dt", [RARE["two_valley"], MANY])
+@pytest.mark.parametrize("n", [63, 1801])
+def test_one_step_launches_of_several_valleys(n, dt, ppl):
+    """two and four per lane: in registers while events are rare, else in LDS"""
+    _run(MODELS["two_valley"], n, 20, dt, ppl, 1)
+
+
+@pytest.mark.parametrize("model,ppl,spl", [("two_valley", 1, 1), ("two_valley", 2, 1), ("two_valley", 4, 1),
+                                           ("si_jacoboni", 1, 1), ("si_jacoboni", 1, 4),
+                                           ("si_jacoboni", 2, 1)])
+def test_fp32_launch_shapes_agree(model, ppl, spl):
+    """the kernels of short launches in FP32 against eight per lane held in LDS
+    for all steps.  The same arithmetic, but the compiler may contract it
+    differently in each kernel: a last bit decides a draw about once in 2^20
+    events, and k differs by a rounding (6e-8) per flight"""
+    from viennaemc_amd import emcgpu
+    spec, n, steps, out = MODELS[model], 5001, 12, []
+    for p, k in ((ppl, spl), (8, steps)):
+        for dt in (RARE[model], MANY):
+            ctx = emcgpu.Context(precision=emcgpu.FP32)
+            ctx.setup(0, spec)
+            ctx.resize([n])
+            ctx.init_particles(0, 11, spec["T"])
+            ctx.step(dt, steps, seed=5, steps_per_launch=k, ppl=p)
+            out.append((ctx.get_particles(0), ctx.averages(0)))
+            ctx.close()
+    for (g, av), (h, bv) in zip(out[:2], out[2:]):
+        same = (g["valley"] == h["valley"]) & (g["sub"] == h["sub"])
+        x, y = g["k"].reshape(-1, 3), h["k"].reshape(-1, 3)
+        # 12 steps of up to about four flights, each rounding twice
+        same &= np.linalg.norm(x - y, axis=1) <= 1e-5 * np.linalg.norm(y, axis=1)
+        # the share of a particle whose 50 events each meet such a draw
+        assert same.mean() > 1 - 1e-3
+        assert np.abs(av["occ"] - bv["occ"]).max() <= 1e-3
+        nv = len(spec["valleys"])
+        cnt = np.array([[np.sum((g["valley"] == v) & (g["sub"] == s)) for s in range(av["sub_occ"].shape[2])]
+                        for v in range(nv)])
+        assert (np.rint(av["sub_occ"][-1] * n) == cnt).all()
+
+
+@pytest.mark.parametrize("n,spl", [(70001, 1), (70001, 3), (70001, 10), (163841, 1), (163841, 10),
+                                   (327681, 1), (327681, 10)])
+@pytest.mark.parametrize("model,dt", [("si_jacoboni", 1e-15), ("two_valley", 1e-15), ("si_jacoboni", 9e-15)])
+def test_tracked_positions_at_every_default(model, dt, n, spl):
+    """positions with one, two and four particles per lane, which follow from
+    the size of the ensemble"""
+    from viennaemc_amd import emcgpu
+    spec, steps, seed = MODELS[model], 10, 21
+    box = np.array([3e-7, 2e-7, 4e-7])
+    M = O.OracleModel(spec)
+    M.set_box(tuple(box))
+    ref = M.init_philox(n, O.thermal_voltage(spec["T"]), seed, positions=True)
+    ctx = emcgpu.Context(precision=emcgpu.FP64)
+    ctx.setup(0, spec)
+    ctx.resize([n])
+    ctx.set_box(0, tuple(box))
+    ctx.set_particles(0, ref["k"], ref["E"], ref["tau"], ref["valley"], ref["sub"])
+    ctx.set_positions(0, ref["pos"])
+    ctx.step(dt, steps, seed=seed, step0=3, steps_per_launch=spl)
+    force, d = field_force(spec)
+    obs = M.run_philox(ref, steps, dt, force, d, seed, step0=3)
+    got, pos = ctx.get_particles(0), ctx.get_positions(0)
+    assert (got["valley"] == ref["valley"]).all() and (got["sub"] == ref["sub"]).all()
+    k, kr = got["k"].reshape(-1, 3), ref["k"].reshape(-1, 3)
+    assert (np.linalg.norm(k - kr, axis=1) <= 1e-12 * np.linalg.norm(kr, axis=1)).all()
+    dp = np.abs(pos - ref["pos"].reshape(-1, 3))
+    assert (np.minimum(dp, box - dp) <= 1e-12 * box).all()
+    av = ctx.averages(0)
+    assert (av["occ"] == obs[:, 2, :len(spec["valleys"])]).all()
+    ctx.close()

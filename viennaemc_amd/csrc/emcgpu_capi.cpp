@@ -668,11 +668,17 @@ emcgpu_status upload_params(emcgpu_ctx *c, double dt_s) {
 // 150k 5.7 / 5.6 / 5.8, 300k 9.0 / 7.3 / 7.4, 400k 11.7 / 9.6 / 7.6, 1M 24.2 /
 // 17.2 / 12.9.  One-step launches in FP64 of models with one valley stream
 // their particles and take eight per lane (screened cooling, 1M: 51.7 us with
-// four, 41.8 with eight).
-int default_ppt(const emcgpu_ctx *c, bool one_step) {
+// four, 41.8 with eight).  With positions they keep one per lane in registers:
+// in FP64 (Si, 1M: 57 us with one, 69 with four in LDS), in FP32 where most
+// particles scatter (10 fs steps, 1M: 52 against 57; at 1 fs 29 against 28).
+int default_ppt(const emcgpu_ctx *c, bool one_step, double events) {
   constexpr long long kFill = 1280 * 64;
-  if (one_step && c->max_v == 1 && c->precision == EMCGPU_FP64 && c->capacity >= 8 * kFill)
-    return 8;
+  if (one_step && c->max_v == 1) {
+    if (c->track_pos && (c->precision == EMCGPU_FP64 || events > 1.0))
+      return 1;
+    if (!c->track_pos && c->precision == EMCGPU_FP64 && c->capacity >= 8 * kFill)
+      return 8;
+  }
   return c->capacity >= 4 * kFill ? 4 : c->capacity >= 2 * kFill ? 2 : 1;
 }
 
@@ -692,8 +698,20 @@ emcgpu_status ensure_partial(emcgpu_ctx *c, int k_steps, int n_tiles) {
   size_t bytes = (size_t)k_steps * partial_per_step(c, n_tiles) * sizeof(double);
   if (bytes > c->partial_bytes) {
     dfreet(c->d_partial);
+    c->partial_bytes = 0;
     HIPCHK(c, hipMalloc((void **)&c->d_partial, bytes));
     c->partial_bytes = bytes;
+  }
+  return EMCGPU_OK;
+}
+
+emcgpu_status ensure_chunks(emcgpu_ctx *c, int k_steps, int n_chunks) {
+  const size_t bytes = (size_t)k_steps * chunks_per_step(c, n_chunks) * sizeof(double);
+  if (bytes > c->chunk_bytes) {
+    dfreet(c->d_chunks);
+    c->chunk_bytes = 0;
+    HIPCHK(c, hipMalloc((void **)&c->d_chunks, bytes));
+    c->chunk_bytes = bytes;
   }
   return EMCGPU_OK;
 }
@@ -840,6 +858,10 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
     return fail(c, EMCGPU_ERR_ARG, "tracked positions run one particle per lane (ppl %d)", ppl);
   StepArgs<R> a;
   fill_common<R>(c, a);
+  for (const auto &in : c->inst)
+    for (size_t v = 0; in.count && v < in.table_mech.size(); v++)
+      if (!in.table_mech[v].empty())
+        a.events = std::max(a.events, s->dt / in.tau0[v]);
   if (baths) {
     a.tally = c->d_tally;
     a.tally_bins = c->tally_bins;
@@ -849,21 +871,26 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
         if (is_scr_hot_kind(m.kind) && m.q_resolved && m.q_resolved_angle)
           a.lds_win = std::max(a.lds_win, 2 * (in.total_bins + (int)in.baths.size()));
   }
-  const int ppt = replay ? 1
-                         : fitting_ppt(a, ppl            ? ppl
-                                          : c->tuned_ppl ? c->tuned_ppl
-                                                         : default_ppt(c, K == 1));
-  const int tile_size = kTile * ppt;
-  const int n_tiles = (int)(c->capacity / tile_size);
+  const int asked = ppl ? ppl : c->tuned_ppl;  // 0: left to the library
+  int ppt = replay ? 1 : fitting_ppt(a, asked ? asked : default_ppt(c, K == 1, a.events));
   long long max_count = 0;
   for (const auto &in : c->inst)
     max_count = std::max<long long>(max_count, (long long)in.count);
-  const int n_chunks = reduce_chunks(max_count, tile_size);
+  int tile_size = 0, n_tiles = 0, n_chunks = 0;
+  auto shape = [&](int p) {
+    ppt = p;
+    tile_size = kTile * ppt;
+    n_tiles = (int)(c->capacity / tile_size);
+    n_chunks = reduce_chunks(max_count, tile_size);
+    return partial_per_step(c, n_tiles) + chunks_per_step(c, n_chunks);
+  };
+  size_t per_step = shape(ppt);
   double *d_partial = nullptr, *d_chunks = nullptr, *d_obs = nullptr;
   if (na) {
     // as many steps per launch as the scratch holds partials for (results
     // do not depend on the launch shape)
-    const size_t per_step = partial_per_step(c, n_tiles) + chunks_per_step(c, n_chunks);
+    if (per_step > na->scratch_len && !asked)
+      per_step = shape(fitting_ppt(a, 8));  // the fewest partials
     const size_t kmax = na->scratch_len / per_step;
     if (kmax < 1)
       return fail(c, EMCGPU_ERR_ARG,
@@ -882,19 +909,21 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
     d_chunks = na->scratch + (size_t)Kr * partial_per_step(c, n_tiles);
     d_obs = na->obs;
   } else {
-    if ((st = ensure_partial(c, Kr, n_tiles)) || (st = ensure_obs(c, s->n_steps)))
+    if ((st = ensure_partial(c, Kr, n_tiles)) || (st = ensure_obs(c, s->n_steps)) ||
+        (st = ensure_chunks(c, Kr, n_chunks)))
       return st;
-    const size_t bytes = (size_t)Kr * chunks_per_step(c, n_chunks) * sizeof(double);
-    if (bytes > c->chunk_bytes) {
-      dfreet(c->d_chunks);
-      HIPCHK(c, hipMalloc((void **)&c->d_chunks, bytes));
-      c->chunk_bytes = bytes;
+    if (reserve_only) {
+      // a later call of one step may take fewer particles per lane
+      if (!replay && !asked) {
+        shape(fitting_ppt(a, default_ppt(c, true, a.events)));
+        if ((st = ensure_partial(c, 1, n_tiles)) || (st = ensure_chunks(c, 1, n_chunks)))
+          return st;
+      }
+      return EMCGPU_OK;
     }
     d_partial = c->d_partial;
     d_chunks = c->d_chunks;
     d_obs = c->h_obs;
-    if (reserve_only)
-      return EMCGPU_OK;
     c->obs_steps = s->n_steps;
   }
 

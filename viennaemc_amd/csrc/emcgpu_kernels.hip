@@ -620,14 +620,13 @@ __global__ __launch_bounds__(kTile, PPT == 1 ? 1 : sizeof(R) == 8 ? 3 : 6) void 
 // filled, so more particles per lane mean fewer idle lanes, and the particles
 // take no LDS.  Used in FP64, whose scatter body is long (screened cooling
 // with 0.13 events per particle and step, 1M: 53.6 -> 41.8 us per step with
-// 8 per lane, 4M: 134.7 -> 106.6), and for small ensembles (50k FP32: 11.9 ->
-// 10.8).  In FP32 the stores of single particles cost more than the passes
-// they save (4M Si: 47.4 us with the particles in LDS, 55.5 streamed).  For
-// models of one valley: with more, the passes' and the stream's registers
+// 8 per lane, 4M: 134.7 -> 106.6), and in FP32 with two per lane.  With more
+// the stores of single particles cost more than the passes they save (4M Si:
+// 47.4 us with the particles in LDS, 55.5 streamed).  For models of one
+// valley without positions: with more, the passes' and the stream's registers
 // do not fit side by side (FP64, two valleys, 8M: 242 us in LDS with 4 per
-// lane, 318 streamed with 8).  With one particle per lane nothing is queued:
-// the particle stays in its lane and the wave stores whole lines at the end
-// (8M Si, FP32 134 -> 121 us, FP64 385 -> 371 against queueing them).
+// lane, 318 streamed with 8; positions: 48 spilled VGPRs, 8M Si 490 us against
+// 377 in registers).
 // ---------------------------------------------------------------------------
 template <typename R>
 constexpr bool streams_one_step(int ppt) {
@@ -637,12 +636,12 @@ constexpr bool streams_one_step(int ppt) {
 constexpr int kOnceQueue = 128;
 constexpr int kOncePass = 60;  // pending events that make a pass worth its while
 
-template <typename R, bool POS>
+template <typename R>
 constexpr size_t once_wave_bytes() {
-  return (size_t)kOnceQueue * ((POS ? 7 : 4) * sizeof(R) + sizeof(uint32_t) + sizeof(uint16_t));
+  return (size_t)kOnceQueue * (4 * sizeof(R) + sizeof(uint32_t) + sizeof(uint16_t));
 }
 
-template <typename R, int PPT, bool HOT, bool POS>
+template <typename R, int PPT, bool HOT>
 __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(StepArgs<R> a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   constexpr int TS = kTile * PPT, Q = kOnceQueue, NV = 1;
@@ -660,8 +659,8 @@ __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(Ste
 
   unsigned char *mem = lds + a.lds_params + a.lds_hot + (size_t)wave * a.lds_wave;
   R *const qx = reinterpret_cast<R *>(mem);
-  R *const qy = qx + Q, *const qz = qy + Q, *const qtau = qz + Q, *const qpos = qtau + Q;
-  uint32_t *const qvs = reinterpret_cast<uint32_t *>(qtau + (POS ? 4 : 1) * Q);
+  R *const qy = qx + Q, *const qz = qy + Q, *const qtau = qz + Q;
+  uint32_t *const qvs = reinterpret_cast<uint32_t *>(qtau + Q);
   uint16_t *const qidx = reinterpret_cast<uint16_t *>(qvs + Q);
   double *const delta = reinterpret_cast<double *>(qidx + Q);  // changes of the counts [n_obs]
   for (int i = lane; i < a.n_obs; i += 64)
@@ -677,7 +676,7 @@ __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(Ste
   const int sub0 = 2 + 3 * a.max_v;
 
   struct Part {
-    R x, y, z, tau, pos[3];
+    R x, y, z, tau;
     uint32_t vs;
     bool valid;
   };
@@ -692,32 +691,21 @@ __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(Ste
       p.z = a.kz[gi];
       p.tau = a.tau[gi];
       p.vs = a.vs[gi];
-      if constexpr (POS) {
-        p.pos[0] = a.px[gi];
-        p.pos[1] = a.py[gi];
-        p.pos[2] = a.pz[gi];
-      }
     }
   };
-  auto store = [&](int i, R x, R y, R z, R E, R tau, const R *pos) {
+  auto store = [&](int i, R x, R y, R z, R E, R tau) {
     const long long gi = base + first + (long long)(i >> 6) * kTile + (i & 63);
     a.kx[gi] = x;
     a.ky[gi] = y;
     a.kz[gi] = z;
     a.E[gi] = E;
     a.tau[gi] = tau;
-    if constexpr (POS) {
-      a.px[gi] = pos[0];
-      a.py[gi] = pos[1];
-      a.pz[gi] = pos[2];
-    }
     return gi;
   };
 
   // the worker lane's particle
   bool busy = false;
   R kx = 0, ky = 0, kz = 0, E = 0, tau = 0, rem = 0;
-  R pos[3] = {0, 0, 0};
   int v = 0, sub = 0, idx = 0;
   uint32_t ev = 0, head = 0, tail = 0;
   int nev = 0, nreal = 0;
@@ -743,11 +731,6 @@ __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(Ste
         const uint32_t vs = qvs[q];
         v = (int)(vs >> 16);
         sub = (int)(vs & 0xffffu);
-        if constexpr (POS) {
-          pos[0] = qpos[q];
-          pos[1] = qpos[Q + q];
-          pos[2] = qpos[2 * Q + q];
-        }
         E = energy_of(kane(v), kx, ky, kz);
         rem = dt - tau;
         ev = 0;
@@ -759,8 +742,8 @@ __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(Ste
       const int v0 = v, sub00 = sub;
       if (busy) {
         rng.pid = (uint32_t)(first + (long long)(idx >> 6) * kTile + (idx & 63));
-        event_once<R, 0, HOT, HOT, POS>(P, kane, a.cum, kx, ky, kz, E, tau, rem, v, sub, ev, rng,
-                                        real, lds_tally, pos);
+        event_once<R, 0, HOT, HOT>(P, kane, a.cum, kx, ky, kz, E, tau, rem, v, sub, ev, rng, real,
+                                   lds_tally);
       }
       nev += (int)__popcll(__ballot(busy));
       nreal += (int)__popcll(__ballot(real));
@@ -769,11 +752,9 @@ __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(Ste
         atomicAdd(delta + sub0 + v * a.max_deg + sub, 1.0);
       }
       if (busy && (!(rem > R(0)) || ev >= kMaxEventsPerStep)) {
-        if constexpr (PPT > 1) {
-          const long long gi = store(idx, kx, ky, kz, E, tau - dt, pos);
-          a.vs[gi] = ((uint32_t)v << 16) | (uint32_t)sub;
-          sums.add(P, kane(v), v, sub, kx, ky, kz, E);
-        }
+        const long long gi = store(idx, kx, ky, kz, E, tau - dt);
+        a.vs[gi] = ((uint32_t)v << 16) | (uint32_t)sub;
+        sums.add(P, kane(v), v, sub, kx, ky, kz, E);
         busy = false;
       }
     }
@@ -796,38 +777,12 @@ __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(Ste
     bool pend = false;
     R en = R(0);
     if (p.valid) {
-      drift<R, POS>(P, kane(vv), (dt < p.tau) ? dt : p.tau, p.x, p.y, p.z, en, 0, ss, p.pos);
+      drift<R>(P, kane(vv), (dt < p.tau) ? dt : p.tau, p.x, p.y, p.z, en, 0, ss);
       pend = dt - p.tau > R(0);
-      if (PPT > 1 && !pend) {
-        store(j * 64 + lane, p.x, p.y, p.z, en, p.tau - dt, p.pos);
+      if (!pend) {
+        store(j * 64 + lane, p.x, p.y, p.z, en, p.tau - dt);
         sums.add(P, kane(vv), vv, ss, p.x, p.y, p.z, en);
       }
-    }
-    if constexpr (PPT == 1) {
-      // one particle per lane: it stays there, and all of a wave's leave at once
-      kx = p.x;
-      ky = p.y;
-      kz = p.z;
-      tau = p.tau;
-      v = vv;
-      sub = ss;
-      idx = lane;
-      if constexpr (POS) {
-        pos[0] = p.pos[0];
-        pos[1] = p.pos[1];
-        pos[2] = p.pos[2];
-      }
-      E = pend ? energy_of(kane(v), kx, ky, kz) : en;
-      rem = dt - tau;
-      busy = pend;
-      passes(1);
-      if (p.valid) {
-        const long long gi = store(lane, kx, ky, kz, E, tau - dt, pos);
-        if (pend)
-          a.vs[gi] = ((uint32_t)v << 16) | (uint32_t)sub;
-        sums.add(P, kane(v), v, sub, kx, ky, kz, E);
-      }
-      break;
     }
     const unsigned long long m = __ballot(pend);
     if (pend) {
@@ -838,11 +793,6 @@ __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(Ste
       qtau[q] = p.tau;
       qvs[q] = p.vs;
       qidx[q] = (uint16_t)(j * 64 + lane);
-      if constexpr (POS) {
-        qpos[q] = p.pos[0];
-        qpos[Q + q] = p.pos[1];
-        qpos[2 * Q + q] = p.pos[2];
-      }
     }
     tail += (uint32_t)__popcll(m);
     wave_lds_fence();
@@ -857,6 +807,180 @@ __global__ __launch_bounds__(kTile, sizeof(R) == 8 ? 3 : 6) void k_bulk_once(Ste
   }
   if constexpr (HOT)
     tally_flush(P, lds_tally, a.tally, a.tally_bins);
+}
+
+// ---------------------------------------------------------------------------
+// production step kernel of short launches: a lane keeps its PPT particles in
+// registers and works through their events itself, one at a time, pulling the
+// state of its next particle that has time left.  No particle passes through
+// LDS, so the first step costs no more than the others and more waves fit a
+// SIMD, while the scatter body runs for as many passes as the wave's busiest
+// lane has events.  Bound by HBM at few events, by vector-ALU issue at many.
+// Which launches take it is keeps_lanes below.
+// ---------------------------------------------------------------------------
+template <typename R, int PPT, bool HOT, bool POS, int NV>
+__global__ __launch_bounds__(kTile) void k_bulk_lanes(StepArgs<R> a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  constexpr int TS = kTile * PPT;
+  const int tile = blockIdx.x;
+  const int inst = tile_instance(a.unit_inst, tile, TS);
+  const InstDev<R> *P = stage_params(lds, a.inst + inst, a.lds_params);
+  uint32_t *lds_tally = reinterpret_cast<uint32_t *>(lds + a.lds_params);
+  if constexpr (HOT)
+    tally_clear(P, lds_tally);
+  const long long base = a.inst_start[inst];
+  const long long count = a.inst_count[inst];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long long first = (long long)tile * TS - base + threadIdx.x;  // local index, j = 0
+
+  R kx[PPT], ky[PPT], kz[PPT], E[PPT], tau[PPT], rem[PPT];
+  R pos[PPT][3];  // POS only
+  int v[PPT], sub[PPT];
+  uint32_t ev[PPT];
+  bool valid[PPT];
+#pragma unroll
+  for (int j = 0; j < PPT; ++j) {
+    const long long local = first + (long long)j * kTile;
+    valid[j] = local < count;
+    kx[j] = ky[j] = kz[j] = E[j] = tau[j] = R(0);
+    pos[j][0] = pos[j][1] = pos[j][2] = R(0);
+    v[j] = sub[j] = 0;
+    if (valid[j]) {
+      const long long gi = base + local;
+      kx[j] = a.kx[gi];
+      ky[j] = a.ky[gi];
+      kz[j] = a.kz[gi];
+      tau[j] = a.tau[gi];
+      const uint32_t vs = a.vs[gi];
+      v[j] = (int)(vs >> 16);
+      sub[j] = (int)(vs & 0xffffu);
+      if constexpr (POS) {
+        pos[j][0] = a.px[gi];
+        pos[j][1] = a.py[gi];
+        pos[j][2] = a.pz[gi];
+      }
+    }
+  }
+  StepRng<R, 0> rng;
+  rng.inst = (uint32_t)inst;
+  rng.k0 = a.key0;
+  rng.k1 = a.key1;
+  const R dt = P->dt;
+  const auto kane = kane_source<R, NV>(P);
+
+  for (int s = 0; s < a.n_steps; ++s) {
+    rng.step = a.step0 + (uint32_t)s;
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) {
+      ev[j] = 0;
+      rem[j] = R(0);
+      if (valid[j]) {
+        // std::min(tau, dt), then tRemaining
+        drift<R, POS>(P, kane(v[j]), (dt < tau[j]) ? dt : tau[j], kx[j], ky[j], kz[j], E[j],
+                      NV == 1 ? 0 : v[j], sub[j], pos[j]);
+        rem[j] = dt - tau[j];
+      }
+    }
+    int nreal = 0;
+    for (;;) {
+      int sel = -1;  // the lane's first particle with time left in the step
+#pragma unroll
+      for (int j = PPT - 1; j >= 0; --j)
+        if (rem[j] > R(0) && ev[j] < kMaxEventsPerStep)
+          sel = j;
+      if (sel < 0)
+        break;
+      R x = kx[0], y = ky[0], z = kz[0], en = E[0], ta = tau[0], rm = rem[0];
+      R wp[3] = {pos[0][0], pos[0][1], pos[0][2]};
+      int vv = v[0], ss = sub[0];
+      uint32_t ee = ev[0];
+#pragma unroll
+      for (int j = 1; j < PPT; ++j)
+        if (sel == j) {
+          x = kx[j];
+          y = ky[j];
+          z = kz[j];
+          en = E[j];
+          ta = tau[j];
+          rm = rem[j];
+          vv = v[j];
+          ss = sub[j];
+          ee = ev[j];
+          if constexpr (POS) {
+            wp[0] = pos[j][0];
+            wp[1] = pos[j][1];
+            wp[2] = pos[j][2];
+          }
+        }
+      rng.pid = (uint32_t)(first + (long long)sel * kTile);
+      event_once<R, 0, HOT, HOT, POS>(P, kane, a.cum, x, y, z, en, ta, rm, vv, ss, ee, rng, nreal,
+                                      lds_tally, wp);
+#pragma unroll
+      for (int j = 0; j < PPT; ++j)
+        if (sel == j) {
+          kx[j] = x;
+          ky[j] = y;
+          kz[j] = z;
+          E[j] = en;
+          tau[j] = ta;
+          rem[j] = rm;
+          v[j] = vv;
+          sub[j] = ss;
+          ev[j] = ee;
+          if constexpr (POS) {
+            pos[j][0] = wp[0];
+            pos[j][1] = wp[1];
+            pos[j][2] = wp[2];
+          }
+        }
+    }
+    int nev = 0;
+    StepSums<R, NV> sums;
+    sums.clear();
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) {
+      nev += (int)ev[j];
+      if (valid[j]) {
+        tau[j] -= dt;
+        sums.add(P, kane(v[j]), v[j], sub[j], kx[j], ky[j], kz[j], E[j]);
+      }
+    }
+    double mine = sums.total(a, wave_sum_i(nev), wave_sum_i(nreal));
+    for (int k = 0; k < a.max_v; ++k) {
+      int n = 0;
+      for (int d = 0; d < a.max_deg; ++d) {
+        int c = 0;
+#pragma unroll
+        for (int j = 0; j < PPT; ++j)
+          c += (int)__popcll(__ballot(valid[j] && v[j] == k && sub[j] == d));
+        n += c;
+        mine = (lane == 2 + 3 * a.max_v + k * a.max_deg + d) ? (double)c : mine;
+      }
+      mine = (lane == 2 + 3 * k) ? (double)n : mine;
+    }
+    if (lane < a.n_obs)
+      a.partial[(((long long)s * a.n_obs + lane) * a.n_tiles + tile) * kSubs + wave] = mine;
+  }
+  if constexpr (HOT)
+    tally_flush(P, lds_tally, a.tally, a.tally_bins);
+
+#pragma unroll
+  for (int j = 0; j < PPT; ++j) {
+    if (valid[j]) {
+      const long long gi = base + first + (long long)j * kTile;
+      a.kx[gi] = kx[j];
+      a.ky[gi] = ky[j];
+      a.kz[gi] = kz[j];
+      a.E[gi] = E[j];
+      a.tau[gi] = tau[j];
+      a.vs[gi] = ((uint32_t)v[j] << 16) | (uint32_t)sub[j];
+      if constexpr (POS) {
+        a.px[gi] = pos[j][0];
+        a.py[gi] = pos[j][1];
+        a.pz[gi] = pos[j][2];
+      }
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1795,12 +1919,50 @@ template int fitting_ppt<float>(StepArgs<float>, int);
 template int fitting_ppt<double>(StepArgs<double>, int);
 
 // the same for the kernel of one-step launches
-template <typename R, bool POS>
+template <typename R>
 size_t once_lds(StepArgs<R> &a) {
-  fused_lds<R, 1, POS>(a);
   a.lds_wave =
-      (int)((once_wave_bytes<R, POS>() + sizeof(double) * (size_t)a.n_obs + 15) & ~size_t(15));
+      (int)((once_wave_bytes<R>() + sizeof(double) * (size_t)a.n_obs + 15) & ~size_t(15));
   return (size_t)a.lds_params + a.lds_hot + (size_t)kSubs * a.lds_wave;
+}
+
+// Launches that keep the particles in the lanes' registers (k_bulk_lanes) where
+// k_bulk_fused would hold them in LDS or k_bulk_once stream them.  us per step
+// here / there, si: one valley of 13 mechanisms, tv: two valleys, 1 fs:
+// - one per lane: up to four steps.  10k FP32 si, 1 / 4 steps: 9.4 / 11.6,
+//   4.5 / 5.0; 8M FP64: si 313 / 368, 214 / 230, tv 279 / 447, 176 / 231; a tie
+//   at 4 steps of tv in FP32 (1M: 13.9 / 13.9).  Where the waves fill the chip
+//   and the registers of k_bulk_fused leave two waves per SIMD, longer ones
+//   too: FP64 tv to 32 steps (8M: 148 / 161; 64 the other way round); with
+//   positions any number (1M si, 64 steps: FP64 30.4 / 38.0, FP32 12.6 / 13.8;
+//   FP32 tv to 8: 13.6 / 13.7)
+// - one step of two or four per lane, several valleys: while events are rare
+//   (at 0.044 expected per particle 4M FP64 100 / 102, 10M 279 / 305, 8M FP32
+//   74 / 84; at 0.088 4M FP64 112 / 109; with baths at 0.2 204 / 170 at 1M;
+//   two per lane in FP64 up to a million particles: 250k 17 / 20, 4M 123 / 116),
+//   always for two in FP32 (4M: 49 / 58, 0.35 events 63 / 76) and with
+//   positions (8M FP64: 283 / 358)
+// - one step with positions of one valley, two per lane (k_bulk_once spills):
+//   300k FP32 20.3 / 21.0
+template <typename R>
+bool keeps_lanes(const StepArgs<R> &a, int ppt) {
+  const bool fp64 = sizeof(R) == 8;
+  if (ppt == 1) {
+    if (a.n_steps <= 4)
+      return true;
+    if ((long long)a.n_tiles * kSubs < 2048)  // two waves on each of the 1024 SIMDs
+      return false;
+    if (a.px)
+      return fp64 || a.max_v == 1 || a.n_steps <= 8;
+    return fp64 && a.max_v > 1 && a.n_steps <= 32;
+  }
+  if (a.n_steps > 1 || ppt > 4)
+    return false;
+  if (a.max_v == 1)
+    return a.px && ppt == 2;
+  if (a.px || (!fp64 && ppt == 2))
+    return true;
+  return a.events < 0.05 && (ppt == 4 || (long long)a.n_tiles * kSubs <= 8192);
 }
 
 template <typename R, int PPT, bool HOT, bool POS>
@@ -1808,11 +1970,20 @@ hipError_t launch_fused(StepArgs<R> a, hipStream_t st) {
   size_t lds = fused_lds<R, PPT, POS>(a);
   const void *f = a.max_v == 1 ? (const void *)k_bulk_fused<R, PPT, HOT, POS, 1>
                                : (const void *)k_bulk_fused<R, PPT, HOT, POS, kMaxV>;
-  if constexpr (streams_one_step<R>(PPT)) {
+  if constexpr (!POS && PPT > 1 && streams_one_step<R>(PPT)) {
     if (a.n_steps == 1 && a.max_v == 1) {
-      lds = once_lds<R, POS>(a);
-      f = (const void *)k_bulk_once<R, PPT, HOT, POS>;
+      lds = once_lds<R>(a);
+      f = (const void *)k_bulk_once<R, PPT, HOT>;
     }
+  }
+  if (keeps_lanes(a, PPT)) {
+    lds = (size_t)a.lds_params + a.lds_hot;
+    if constexpr (PPT == 1 || (PPT == 2 && POS))
+      if (a.max_v == 1)
+        f = (const void *)k_bulk_lanes<R, PPT, HOT, POS, 1>;
+    if constexpr (PPT <= 4)
+      if (a.max_v > 1)
+        f = (const void *)k_bulk_lanes<R, PPT, HOT, POS, kMaxV>;
   }
   if (lds > kMaxBulkLds)
     return hipErrorInvalidValue;
