@@ -1536,6 +1536,8 @@ emcgpu_status emcgpu_set_model(emcgpu_ctx *c, int instance, const emcgpu_valley_
     for (const auto &d : i2.valleys)
       md = std::max(md, d.degeneracy);
   }
+  if (mv != c->max_v || md != c->max_deg)
+    c->obs_steps = 0;  // the last call's sums have the old layout
   c->max_v = mv;
   c->max_deg = md;
   c->n_obs = 2 + mv * (3 + md);
