@@ -716,16 +716,36 @@ emcgpu_status ensure_chunks(emcgpu_ctx *c, int k_steps, int n_chunks) {
   return EMCGPU_OK;
 }
 
+void free_obs(double *p, bool pinned) {
+  if (pinned)
+    (void)hipHostFree(p);
+  else
+    (void)hipFree(p);
+}
+
+// the step sums of n_steps steps: pinned host memory up to kKeepBytes, device
+// memory beyond.  The sums of the last call stay readable until the next call
+// writes its own, also if no memory is left for the larger buffer.
 emcgpu_status ensure_obs(emcgpu_ctx *c, int n_steps) {
-  size_t bytes = (size_t)c->n_inst * n_steps * c->n_obs * sizeof(double);
-  if (bytes > c->obs_bytes) {
-    // an earlier call's launches may still write the old buffer
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    hfreet(c->h_obs);
-    c->obs_bytes = 0;
-    HIPCHK(c, hipHostMalloc((void **)&c->h_obs, bytes, hipHostMallocDefault));
-    c->obs_bytes = bytes;
+  const size_t step = (size_t)c->n_inst * c->n_obs * sizeof(double), bytes = step * n_steps;
+  if (bytes <= c->obs_bytes)
+    return EMCGPU_OK;
+  const bool pinned = bytes <= kKeepBytes;
+  double *p = nullptr;
+  HIPCHK(c, pinned ? hipHostMalloc((void **)&p, bytes, hipHostMallocDefault)
+                   : hipMalloc((void **)&p, bytes));
+  // an earlier call's launches may still write the old buffer
+  hipError_t e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess && c->obs_steps > 0)
+    e = hipMemcpy(p, c->obs, step * c->obs_steps, hipMemcpyDefault);
+  if (e != hipSuccess) {
+    free_obs(p, pinned);
+    HIPCHK(c, e);
   }
+  free_obs(c->obs, c->obs_pinned);
+  c->obs = p;
+  c->obs_pinned = pinned;
+  c->obs_bytes = bytes;
   return EMCGPU_OK;
 }
 
@@ -923,7 +943,7 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
     }
     d_partial = c->d_partial;
     d_chunks = c->d_chunks;
-    d_obs = c->h_obs;
+    d_obs = c->obs;
     c->obs_steps = s->n_steps;
   }
 
@@ -1421,7 +1441,7 @@ void emcgpu_destroy(emcgpu_ctx *c) {
   dfree(c->d_cum);
   dfreet(c->d_partial);
   dfreet(c->d_chunks);
-  hfreet(c->h_obs);
+  free_obs(c->obs, c->obs_pinned);
   hfreet(c->stage);
   dfree(c->work);
   dfreet(c->d_obs0);
@@ -2607,8 +2627,12 @@ emcgpu_status emcgpu_get_observables(const emcgpu_ctx *c0, int instance, double 
   if (out && c->obs_steps > 0 && c->device >= 0) {
     (void)hipSetDevice(c->device);
     const size_t m = (size_t)c->obs_steps * c->n_obs;
+    const double *const src = c->obs + (size_t)instance * m;
+    if (!c->obs_pinned)
+      HIPCHK(c, hipMemcpyAsync(out, src, m * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    std::memcpy(out, c->h_obs + (size_t)instance * m, m * sizeof(double));
+    if (c->obs_pinned)
+      std::memcpy(out, src, m * sizeof(double));
   }
   return EMCGPU_OK;
 }

@@ -106,9 +106,10 @@ struct emcgpu_ctx {
   double *d_chunks = nullptr;  // (sum, compensation) pairs of the first reduction pass
   size_t chunk_bytes = 0;
   // per-step sums of the last call [instance][step][value], in pinned host
-  // memory that the reduction kernels write: a read waits for the stream and
-  // copies nothing from the device
-  double *h_obs = nullptr;
+  // memory that the reduction kernels write (a read waits for the stream and
+  // copies nothing from the device), or in device memory beyond kKeepBytes
+  double *obs = nullptr;
+  bool obs_pinned = true;
   // of the calls on host arrays, kept up to kKeepBytes each and freed with the
   // context: device workspace, pinned staging of particle transfers
   void *work = nullptr;
@@ -155,8 +156,10 @@ struct emcgpu_ctx {
 #define HIPCHK(c, x)                                                                     \
   do {                                                                                   \
     hipError_t e_ = (x);                                                                 \
-    if (e_ != hipSuccess)                                                                \
+    if (e_ != hipSuccess) {                                                              \
+      (void)hipGetLastError(); /* not the next launch's error */                         \
       return fail((c), EMCGPU_ERR_HIP, "%s failed: %s", #x, hipGetErrorString(e_));      \
+    }                                                                                    \
   } while (0)
 
 namespace emcgpu {
@@ -178,8 +181,10 @@ inline emcgpu_status fail(emcgpu_ctx *c, emcgpu_status st, const char *fmt, ...)
 #define HIPCHK(c, x)                                                                     \
   do {                                                                                   \
     hipError_t e_ = (x);                                                                 \
-    if (e_ != hipSuccess)                                                                \
+    if (e_ != hipSuccess) {                                                              \
+      (void)hipGetLastError(); /* not the next launch's error */                         \
       return fail((c), EMCGPU_ERR_HIP, "%s failed: %s", #x, hipGetErrorString(e_));      \
+    }                                                                                    \
   } while (0)
 
 inline size_t real_size(const emcgpu_ctx *c) {
