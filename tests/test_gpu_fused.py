@@ -170,3 +170,34 @@ def test_tracked_positions_at_every_default(model, dt, n, spl):
     av = ctx.averages(0)
     assert (av["occ"] == obs[:, 2, :len(spec["valleys"])]).all()
     ctx.close()
+
+
+def test_two_threads_with_workgroups_of_different_lds():
+    """contexts of different models step side by side in the same kernel, each
+    with its own amount of LDS above 64 KB"""
+    import threading
+    from viennaemc_amd import emcgpu
+    names, n, calls = ("si_jacoboni", "para_iso"), 4096, 40
+
+    def run(name, out):
+        ctx = emcgpu.Context(precision=emcgpu.FP64)
+        ctx.setup(0, MODELS[name])
+        ctx.resize([n])
+        ctx.init_particles(0, 2, 300.0)
+        for c in range(calls):
+            ctx.step(1e-15, 8, seed=6, step0=8 * c, steps_per_launch=8, ppl=8)
+        out[name] = (ctx.get_particles(0), ctx.observables(0))
+        ctx.close()
+
+    alone, together = {}, {}
+    for name in names:
+        run(name, alone)
+    threads = [threading.Thread(target=run, args=(name, together)) for name in names]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for name in names:
+        (p, obs), (q, want) = together[name], alone[name]
+        assert all(np.array_equal(p[key], q[key]) for key in p)
+        assert np.array_equal(obs, want)

@@ -1988,8 +1988,10 @@ hipError_t launch_fused(StepArgs<R> a, hipStream_t st) {
   if (lds > kMaxBulkLds)
     return hipErrorInvalidValue;
   if (lds > 64 * 1024) {
+    // the limit is the kernel's, not the launch's: every context sets the same
+    // one, whichever thread comes between this call and the launch
     const hipError_t e =
-        hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxBulkLds);
     if (e != hipSuccess)
       return e;
   }
