@@ -340,6 +340,28 @@ def test_self_consistent_run(precision):
     ctx.close()
 
 
+@pytest.mark.parametrize("nx,ny", [(12, 7), (82, 9), (83, 41), (162, 17), (163, 18), (194, 85), (194, 86)])
+def test_separable_corrections_of_every_shape(nx, ny):
+    """the separable inverse where its kernels change: 10 to 192 active
+    columns in slices of few rows, of up to 20 and of more; 255 and 258
+    workgroups.  It is exact, so one correction meets the stopping rule at
+    (almost) every step, with the potential of the multigrid solves"""
+    emcgpu = _emc()
+    dev = resistor_device(nx=nx, ny=ny, n_particles=20_000, contact_nodes=max(3, nx // 20))
+    res = {}
+    for mode in (emcgpu.POISSON_MULTIGRID, emcgpu.POISSON_AUTO):
+        ctx = _ctx(dev=dev, precision=emcgpu.FP64, tol=1e-10)
+        ctx.device_init(77)
+        out = ctx.device_step(0.1e-15, 10, seed=77, poisson_mode=mode)
+        assert (out["poisson_resid"] <= 1e-10).all()
+        res[mode] = (out["poisson_iters"][1:], ctx.device_fields()["pot"])
+        ctx.close()
+    work, pot = res[emcgpu.POISSON_AUTO]
+    ref = res[emcgpu.POISSON_MULTIGRID][1]
+    assert (work <= 1).mean() >= 0.8
+    assert np.abs(pot - ref).max() < 1e-8 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("precision", [0, 1])
 def test_dense_poisson_corrections_match_multigrid(precision):
     """The per-step solves with Newton corrections from an inverse of the

@@ -2369,25 +2369,35 @@ hipError_t dev_green_lds(size_t lds) {
 // Newton correction by the separable inverse.  Both launches run a block per
 // (active row j, chunk of kFdChunk columns) and are bound by the latency of
 // dependent L2 round trips, so the loads that depend on nothing are issued
-// first (the x transform's matrix, before the flags are even read), every
-// sum keeps up to twenty-four loads in flight per lane and is split over as
-// many threads as the block has: the row of the y transform (all mx columns,
-// in LDS) takes P = kFdThreads / mx threads per column, each summing a P-th
-// of the rows; the chunk's x sums take one lane per output column and the
-// block's waves each a slice of the rows.  On 198 x 50 active nodes the two
-// take 8.4 and 8.3 us (9.6 and 9.0 with eight loads at a time, all of them
-// after the flags)
+// first (AHEAD rows of a wave's slice of the x transform's matrix, before the
+// flags are even read), every sum keeps up to ROWS loads in flight per lane
+// and is split over as many threads as the block has: the row of the y
+// transform (all mx columns, in LDS) takes P = kFdThreads / mx threads per
+// column, each summing a P-th of the rows; the chunk's x sums take one lane
+// per output column and the block's waves each a slice of the rows.  The order
+// of the additions does not depend on AHEAD and ROWS.
+//
+// us forward / backward with eight loads and none ahead (72 VGPRs), <32, 24>
+// (174, one block per CU), <16, 16> (128, two): 200 x 50 nodes 9.8 / 8.5, 9.1 /
+// 8.4, 10.0 / 8.6; 250 x 64 (248 blocks) 12.1 / 10.7, 10.8 / 9.4, 12.3 / 10.6;
+// 250 x 66 (256 CUs do not hold 264 blocks of <32, 24>) 15.4 / 13.6, 17.5 /
+// 16.2, 14.4 / 13.0; 150 x 140 16.0 / 14.5, 21.2 / 18.7, 15.8 / 13.9; 400 x 200
+// 123 / 110, 136 / 124, 122 / 108; 126 x 101 11.3 / 9.5, 11.8 / 9.8, 10.8 / 8.8;
+// 160 x 48 7.8 / 7.3, 7.8 / 7.4, 7.5 / 7.1.  A slice of up to 80 columns has at
+// most ten rows, which <32, 24> pads to 32: 50 x 20 5.9 / 5.6, 6.7 / 6.3, and
+// <8, 8> 5.7 / 5.5; 80 x 100 9.9 / 8.7, 10.4 / 9.0, 9.8 / 8.4
 constexpr int kFdChunk = 64;
 constexpr int kFdWaves = kFdThreads / 64;
-constexpr int kFdAhead = 32;  // rows of a wave's slice held in registers
+constexpr unsigned kFdAlone = 256;  // blocks that have a CU each
 
 // rows [r0, r1) of the x transform's matrix for one output column: the first
-// kFdAhead in registers
+// AHEAD in registers
+template <int AHEAD>
 struct FdSlice {
   const double *m;
   size_t ld;
   int r0, r1;
-  double x[kFdAhead];
+  double x[AHEAD > 0 ? AHEAD : 1];
   __device__ __forceinline__ FdSlice(const double *M, int mx, int k) {
     const int w = (int)threadIdx.x >> 6;
     const int span = (mx + kFdWaves - 1) / kFdWaves;
@@ -2396,7 +2406,7 @@ struct FdSlice {
     r0 = w * span;
     r1 = k < mx ? min(mx, r0 + span) : 0;
 #pragma unroll
-    for (int u = 0; u < kFdAhead; ++u)
+    for (int u = 0; u < AHEAD; ++u)
       x[u] = r0 + u < r1 ? m[(size_t)(r0 + u) * ld] : 0.0;
   }
   // sum over the slice of m[r][k] row[r]: eight rows at a time into four
@@ -2406,7 +2416,7 @@ struct FdSlice {
     if (r0 >= r1)
       return 0.0;
 #pragma unroll
-    for (int g = 0; g < kFdAhead; g += 8) {
+    for (int g = 0; g < AHEAD; g += 8) {
       if (r0 + g + 8 <= r1) {
 #pragma unroll
         for (int u = 0; u < 8; ++u)
@@ -2418,7 +2428,7 @@ struct FdSlice {
             s[0] = fma(x[g + u], row[r0 + g + u], s[0]);
       }
     }
-    int r = r0 + kFdAhead;
+    int r = r0 + AHEAD;
     for (; r + 8 <= r1; r += 8) {
       double y[8];
 #pragma unroll
@@ -2435,8 +2445,8 @@ struct FdSlice {
 };
 
 // row[q] = sum_b w[b] in(b, q) for the mx columns q, P threads per column
-// (part: max(mx, kFdThreads) doubles of LDS)
-template <typename IN>
+// (part: max(mx, kFdThreads) doubles of LDS), ROWS loads in flight
+template <int ROWS, typename IN>
 __device__ __forceinline__ void fd_row(const double *w, int my, int mx, double *row, double *part,
                                        IN in) {
   const int P = max(1, min(kFdThreads / mx, 8));
@@ -2446,13 +2456,13 @@ __device__ __forceinline__ void fd_row(const double *w, int my, int mx, double *
     const int b0 = p * span, b1 = min(my, b0 + span);
     double s[4] = {0.0, 0.0, 0.0, 0.0};
     int b = b0;
-    for (; b + 24 <= b1; b += 24) {
-      double x[24];
+    for (; ROWS > 8 && b + ROWS <= b1; b += ROWS) {
+      double x[ROWS];
 #pragma unroll
-      for (int u = 0; u < 24; ++u)
+      for (int u = 0; u < ROWS; ++u)
         x[u] = in(b + u, q);
 #pragma unroll
-      for (int u = 0; u < 24; ++u)
+      for (int u = 0; u < ROWS; ++u)
         s[u & 3] = fma(w[b + u], x[u], s[u & 3]);
     }
     for (; b + 8 <= b1; b += 8) {
@@ -2480,7 +2490,8 @@ __device__ __forceinline__ void fd_row(const double *w, int my, int mx, double *
 
 // the chunk's x sums: out = sum_r M[r][k] row[r] for lane k of the chunk,
 // each wave a slice of the rows; the result is valid in wave 0
-__device__ __forceinline__ double fd_chunk(const FdSlice &M, const double *row, double *part) {
+template <int AHEAD>
+__device__ __forceinline__ double fd_chunk(const FdSlice<AHEAD> &M, const double *row, double *part) {
   const int w = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
   part[w * kFdChunk + lane] = M.dot(row);
   __syncthreads();
@@ -2492,18 +2503,19 @@ __device__ __forceinline__ double fd_chunk(const FdSlice &M, const double *row, 
 }
 
 // t[j][k] = sum_q Px[k][q] (sum_b Py[j][b] F[b][q]) / (lx[k] + ly[j])
-__global__ __launch_bounds__(kFdThreads) void k_fd_fwd(GreenArgs a, int c) {
+template <int AHEAD, int ROWS>
+__global__ __launch_bounds__(kFdThreads, AHEAD > 16 ? 2 : 4) void k_fd_fwd(GreenArgs a, int c) {
   extern __shared__ double fd_lds[];  // [mx] row, [max(mx, kFdThreads)] partial sums
   if (a.interval > 1 && a.state->step % a.interval != 0)
     return;
   const FdOps &f = a.fd;
   const int j = blockIdx.y, mx = f.mx, my = f.my, nx = a.nx;
   const int k = (int)blockIdx.x * kFdChunk + ((int)threadIdx.x & 63);
-  const FdSlice M(f.pxt, mx, k);
+  const FdSlice<AHEAD> M(f.pxt, mx, k);
   if (*a.flag == (unsigned long long)a.state->step + 1ull || green_converged(a, c))
     return;
   double *row = fd_lds, *part = fd_lds + mx;
-  fd_row(f.py + (size_t)j * my, my, mx, row, part,
+  fd_row<ROWS>(f.py + (size_t)j * my, my, mx, row, part,
          [&](int b, int q) { return a.g[(size_t)f.iy[b] * nx + f.ix[q]]; });
   const double t = fd_chunk(M, row, part);
   if (threadIdx.x < 64 && k < mx)
@@ -2511,22 +2523,29 @@ __global__ __launch_bounds__(kFdThreads) void k_fd_fwd(GreenArgs a, int c) {
 }
 
 // pot[j][q] += sum_k Bx[q][k] (sum_l By[j][l] t[l][k])
-__global__ __launch_bounds__(kFdThreads) void k_fd_bwd(GreenArgs a, int c) {
+template <int AHEAD, int ROWS>
+__global__ __launch_bounds__(kFdThreads, AHEAD > 16 ? 2 : 4) void k_fd_bwd(GreenArgs a, int c) {
   extern __shared__ double fd_lds[];  // [mx] row, [max(mx, kFdThreads)] partial sums
   if (a.interval > 1 && a.state->step % a.interval != 0)
     return;
   const FdOps &f = a.fd;
   const int j = blockIdx.y, mx = f.mx, my = f.my;
   const int q = (int)blockIdx.x * kFdChunk + ((int)threadIdx.x & 63);
-  const FdSlice M(f.bxt, mx, q);
+  const FdSlice<AHEAD> M(f.bxt, mx, q);
   if (*a.flag == (unsigned long long)a.state->step + 1ull || green_converged(a, c))
     return;
   double *row = fd_lds, *part = fd_lds + mx;
-  fd_row(f.by + (size_t)j * my, my, mx, row, part,
+  fd_row<ROWS>(f.by + (size_t)j * my, my, mx, row, part,
          [&](int l, int k) { return f.t[(size_t)l * mx + k]; });
   const double x = fd_chunk(M, row, part);
   if (threadIdx.x < 64 && q < mx)
     a.pot[(size_t)f.iy[j] * a.nx + f.ix[q]] += x;
+}
+
+template <int AHEAD, int ROWS>
+void launch_fd(const GreenArgs &a, int it, dim3 grid, size_t lds, hipStream_t st) {
+  hipLaunchKernelGGL((k_fd_fwd<AHEAD, ROWS>), grid, dim3(kFdThreads), lds, st, a, it);
+  hipLaunchKernelGGL((k_fd_bwd<AHEAD, ROWS>), grid, dim3(kFdThreads), lds, st, a, it);
 }
 
 // residual check, correction (skipped once a check meets the stopping
@@ -2538,8 +2557,12 @@ hipError_t dev_launch_green(const GreenArgs &a, int iters, int blocks, hipStream
     if (a.use_fd) {
       const size_t lds = (size_t)(a.fd.mx + max(a.fd.mx, kFdThreads)) * sizeof(double);
       const dim3 grid((unsigned)((a.fd.mx + kFdChunk - 1) / kFdChunk), (unsigned)a.fd.my);
-      hipLaunchKernelGGL(k_fd_fwd, grid, dim3(kFdThreads), lds, st, a, it);
-      hipLaunchKernelGGL(k_fd_bwd, grid, dim3(kFdThreads), lds, st, a, it);
+      if (a.fd.mx <= 80)
+        launch_fd<8, 8>(a, it, grid, lds, st);
+      else if (a.fd.mx > 160 && grid.x * grid.y <= kFdAlone)
+        launch_fd<32, 24>(a, it, grid, lds, st);
+      else
+        launch_fd<16, 16>(a, it, grid, lds, st);
     } else {
       hipLaunchKernelGGL(k_green_apply, dim3((unsigned)blocks), dim3(kGreenThreads),
                          (size_t)a.ld * sizeof(float), st, a, it);
