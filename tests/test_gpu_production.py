@@ -277,3 +277,38 @@ def test_batched_instances_are_independent():
         g = ctx.get_particles(i)
         assert (g["valley"] == ref["valley"]).all() and (g["sub"] == ref["sub"]).all()
         assert _rel_k(g["k"].reshape(-1, 3), ref["k"].reshape(-1, 3)).max() < REL_TOL
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_field_step_and_tables_changed_between_calls(precision):
+    """a context whose field, time step and tables change from call to call
+    against contexts that are set up with them: bit-identical"""
+    import copy
+    emcgpu = _emc()
+    base = MODELS["si_jacoboni"]
+    other = copy.deepcopy(base)
+    other["mechs"] = other["mechs"][:5]
+    n, state = 777, None
+    ctx = _ctx("si_jacoboni", n, precision)
+    ctx.init_particles(0, 9, 300.0)
+    # (model, field, dt): the tables change with the model only
+    for i, (spec, kv, dt) in enumerate([(base, 10, 1e-15), (base, 50, 1e-15), (base, 50, 2e-15),
+                                        (other, 50, 2e-15), (other, 20, 2e-15), (base, 20, 1e-15)]):
+        spec = dict(spec, field_kvcm=kv)
+        fresh = emcgpu.Context(precision=precision)
+        fresh.setup(0, spec)
+        fresh.resize([n])
+        if i == 0 or spec["mechs"] is not last["mechs"]:
+            ctx.setup(0, spec)
+        else:
+            ctx.set_field(0, spec["field_dir"], kv * 1e5)
+        last = spec
+        state = ctx.get_particles(0)
+        for c in (ctx, fresh):
+            c.set_particles(0, state["k"], state["E"], state["tau"], state["valley"], state["sub"])
+            c.step(dt, 9, seed=4, step0=9 * i)
+        g, f = ctx.get_particles(0), fresh.get_particles(0)
+        assert all(np.array_equal(g[key], f[key]) for key in g)
+        assert np.array_equal(ctx.observables(0), fresh.observables(0))
+        fresh.close()
+    ctx.close()

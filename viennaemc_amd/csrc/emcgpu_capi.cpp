@@ -599,50 +599,62 @@ emcgpu_status upload_params(emcgpu_ctx *c, double dt_s) {
       return st;
   }
   std::vector<InstDev<R>> P(c->n_inst);
+  // tables that are neither new nor rebuilt on the GPU are there already (a new
+  // field or time step: 64 models of 2000 levels x 13 tables are 20 MB in FP64,
+  // 2.4 of the 2.6 ms that new fields and the step after them took)
+  bool tables = c->tables_dirty || c->n_baths > 0;
+  for (const Instance &in : c->inst)
+    tables = tables || in.plasma();
   std::vector<R> cum;
   size_t cum64_elems = 0;  // FP64 copies of the tables that are rebuilt on the GPU
   size_t total = 0;
   for (const Instance &in : c->inst)
     for (size_t v = 0; in.has_tables && v < in.valleys.size(); v++)
       total += (size_t)in.n_levels * row_stride((int)in.table_mech[v].size());
-  cum.reserve(total);
+  if (tables)
+    cum.reserve(total);
   for (int i = 0; i < c->n_inst; i++) {
-    const Instance &in = c->inst[i];
-    std::vector<long long> off(kMaxV, 0), off64(kMaxV, 0);
+    Instance &in = c->inst[i];
     if (!in.has_tables)
       continue;
-    for (size_t v = 0; v < in.valleys.size(); v++) {
-      off[v] = (long long)cum.size();
-      off64[v] = (long long)cum64_elems;
-      const int nt = (int)in.table_mech[v].size();
-      const int head = row_head(nt), stride = row_stride(nt);
-      const size_t nl = (size_t)in.n_levels;
-      cum.resize(cum.size() + nl * stride, (R)kRowPad);
-      R *const rows = cum.data() + off[v];
-      const double *const src = in.cum[v].data();
-      for (size_t l = 0; l < nl; l++)
-        for (int j = 0; j < nt; j++)
-          rows[l * stride + head + j] = (R)src[j * nl + l];
-      for (int g = 0; head && g < row_groups(nt); g++) {
-        const int end = std::min(4 * g + 3, nt - 1);
+    if (tables) {
+      std::vector<long long> off(kMaxV, 0), off64(kMaxV, 0);
+      for (size_t v = 0; v < in.valleys.size(); v++) {
+        off[v] = (long long)cum.size();
+        off64[v] = (long long)cum64_elems;
+        const int nt = (int)in.table_mech[v].size();
+        const int head = row_head(nt), stride = row_stride(nt);
+        const size_t nl = (size_t)in.n_levels;
+        cum.resize(cum.size() + nl * stride, (R)kRowPad);
+        R *const rows = cum.data() + off[v];
+        const double *const src = in.cum[v].data();
         for (size_t l = 0; l < nl; l++)
-          rows[l * stride + g] = rows[l * stride + head + end];
+          for (int j = 0; j < nt; j++)
+            rows[l * stride + head + j] = (R)src[j * nl + l];
+        for (int g = 0; head && g < row_groups(nt); g++) {
+          const int end = std::min(4 * g + 3, nt - 1);
+          for (size_t l = 0; l < nl; l++)
+            rows[l * stride + g] = rows[l * stride + head + end];
+        }
+        cum64_elems += nl * nt;
       }
-      cum64_elems += nl * nt;
+      in.cum_off = off64;
+      in.tab_off = off;
     }
-    c->inst[i].cum_off = off64;
-    c->inst[i].tab_off = off;
-    lower_instance<R>(c, in, dt_s, P[i], off);
+    lower_instance<R>(c, in, dt_s, P[i], in.tab_off);
   }
-  if (cum.empty())
-    cum.push_back(R(0));
-  size_t bytes = cum.size() * sizeof(R);
-  if (bytes > c->cum_bytes) {
-    dfree(c->d_cum);
-    HIPCHK(c, hipMalloc(&c->d_cum, bytes));
-    c->cum_bytes = bytes;
+  if (tables) {
+    if (cum.empty())
+      cum.push_back(R(0));
+    size_t bytes = cum.size() * sizeof(R);
+    if (bytes > c->cum_bytes) {
+      dfree(c->d_cum);
+      c->cum_bytes = 0;
+      HIPCHK(c, hipMalloc(&c->d_cum, bytes));
+      c->cum_bytes = bytes;
+    }
+    HIPCHK(c, hipMemcpyAsync(c->d_cum, cum.data(), bytes, hipMemcpyHostToDevice, c->stream));
   }
-  HIPCHK(c, hipMemcpyAsync(c->d_cum, cum.data(), bytes, hipMemcpyHostToDevice, c->stream));
   if (!c->d_params)
     HIPCHK(c, hipMalloc(&c->d_params, sizeof(InstDev<R>) * c->n_inst));
   HIPCHK(c, hipMemcpyAsync(c->d_params, P.data(), sizeof(InstDev<R>) * c->n_inst,
@@ -652,7 +664,7 @@ emcgpu_status upload_params(emcgpu_ctx *c, double dt_s) {
   emcgpu_status st = upload_rebuild<R>(c, cum64_elems);
   if (st)
     return st;
-  c->params_dirty = false;
+  c->params_dirty = c->tables_dirty = false;
   c->params_dt = dt_s;
   return EMCGPU_OK;
 }
@@ -1178,7 +1190,7 @@ emcgpu_status finish_tables(emcgpu_ctx *c, Instance &in, int n_levels, double ma
     in.cum[v] = std::move(t);
   }
   in.has_tables = true;
-  c->params_dirty = true;
+  c->params_dirty = c->tables_dirty = true;
   return EMCGPU_OK;
 }
 
@@ -1561,7 +1573,7 @@ emcgpu_status emcgpu_set_model(emcgpu_ctx *c, int instance, const emcgpu_valley_
   c->max_v = mv;
   c->max_deg = md;
   c->n_obs = 2 + mv * (3 + md);
-  c->params_dirty = true;
+  c->params_dirty = c->tables_dirty = true;
   return EMCGPU_OK;
 }
 
@@ -2165,7 +2177,7 @@ emcgpu_status emcgpu_set_screening(emcgpu_ctx *c, int instance, const emcgpu_scr
   if (was != in.plasma())
     in.has_tables = false;
   in.dev_scr = false;
-  c->params_dirty = true;
+  c->params_dirty = c->tables_dirty = true;
   return EMCGPU_OK;
 }
 
@@ -2219,7 +2231,7 @@ emcgpu_status emcgpu_update_screening(emcgpu_ctx *c, int instance) {
     return st;
   // the next upload lowers the new q_s^2 and rebuilds the tables and the
   // window sums on the GPU from it
-  c->params_dirty = true;
+  c->params_dirty = c->tables_dirty = true;
   const double dt = c->params_dt > 0 ? c->params_dt : 1e-15;
   return c->precision == EMCGPU_FP32 ? upload_params<float>(c, dt) : upload_params<double>(c, dt);
 }
@@ -2290,7 +2302,7 @@ emcgpu_status emcgpu_set_baths(emcgpu_ctx *c, int instance, const emcgpu_bath_de
   if (in.has_hot)
     in.has_tables = false;  // the hot-phonon rates read the new baths
   c->bath_layout_dirty = true;
-  c->params_dirty = true;
+  c->params_dirty = c->tables_dirty = true;
   return EMCGPU_OK;
 }
 
@@ -2352,7 +2364,7 @@ emcgpu_status emcgpu_set_bath_state(emcgpu_ctx *c, int instance, int bath, const
                         hipMemcpyHostToDevice));
   }
   // the tables follow the new state on the next step
-  c->params_dirty = true;
+  c->params_dirty = c->tables_dirty = true;
   return EMCGPU_OK;
 }
 

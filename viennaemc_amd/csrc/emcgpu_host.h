@@ -97,7 +97,8 @@ struct emcgpu_ctx {
   void *d_params = nullptr;
   void *d_cum = nullptr;
   size_t cum_bytes = 0;
-  bool params_dirty = true;
+  bool params_dirty = true;  // the parameter blocks on the device are stale
+  bool tables_dirty = true;  // so are the tables
   double params_dt = 0;
   // observables
   int max_v = 1, max_deg = 1, n_obs = 0;
