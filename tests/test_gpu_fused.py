@@ -80,10 +80,18 @@ def test_table_rows(nt):
 @pytest.mark.parametrize("ppl", [1, 2, 4, 8])
 @pytest.mark.parametrize("model,dt", [("screened_polar", 0.5e-15), ("two_valley", 15e-15)])
 def test_one_step_launches(model, dt, ppl):
-    """the streaming kernel of one-step launches: waves whose particles come
-    in one to eight chunks of 64, the last one ragged, with few and with
-    mostly scattering particles"""
+    """one-step launches with few events (one valley: streamed in one to eight
+    chunks of 64, the last one ragged; in registers with one per lane) and with
+    mostly scattering particles (two valleys: held in LDS)"""
     _run(MODELS[model], 1801, 12, dt, ppl, 1)
+
+
+@pytest.mark.parametrize("ppl", [2, 4, 8])
+@pytest.mark.parametrize("n", [127, 1801, 4097])
+def test_streaming_with_many_events(n, ppl):
+    """most particles of a chunk wait when the next 64 arrive: the queue holds
+    up to 59 + 64 of its 128 entries and wraps"""
+    _run(MODELS["si_jacoboni"], n, 8, 15e-15, ppl, 1)
 
 
 # dt such that about 4 % and most of the particles scatter in a step
