@@ -194,7 +194,10 @@ typedef struct {
   int timing;           /* non-zero: time every launch with HIP events */
   int particles_per_lane; /* production kernel: particles owned by each
                              GPU lane, 1, 2, 4 or 8 (0 = the value of
-                             emcgpu_autotune, else the library default) */
+                             emcgpu_autotune, else the library default);
+                             fewer run where baths of many bins leave a
+                             workgroup too little LDS.  Results do not
+                             depend on it */
   int use_graph;        /* production: capture the call's launches (step and
                            reduction kernels) in a HIP graph and launch it;
                            the executable graph is updated in place on the
@@ -301,7 +304,8 @@ emcgpu_status emcgpu_init_particles_energy(emcgpu_ctx *ctx, int instance,
  * flight (include/emcParticleDrift.hpp:26-34) and wrapped into the device
  * box [0, maxPos] (basicBulkParticleHandler.hpp:600-613); it is written by
  * print (:227-248).  emcgpu_set_box turns this on for the context (the
- * steps then take particles_per_lane 0 or 1 only) with the instance's box
+ * steps then take particles_per_lane 0, the library's choice of 1, 2 or 4
+ * by the size of the ensemble, or 1) with the instance's box
  * max_pos[3] [m]; emcgpu_init_particles then also draws positions uniform
  * in the box.  Positions are [n][3] in m. */
 emcgpu_status emcgpu_set_box(emcgpu_ctx *ctx, int instance, const double max_pos[3]);

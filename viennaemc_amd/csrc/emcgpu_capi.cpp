@@ -884,10 +884,10 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
   } else if (!reserve_only) {
     c->bath_hist_steps = 0;
   }
-  // particles per lane of the production kernel (replay and tracked
-  // positions: the caller asks for none or one per lane)
+  // particles per lane of the production kernel; with tracked positions the
+  // caller leaves them to the library or asks for one
   if (c->track_pos && ppl > 1)
-    return fail(c, EMCGPU_ERR_ARG, "tracked positions run one particle per lane (ppl %d)", ppl);
+    return fail(c, EMCGPU_ERR_ARG, "tracked positions take particles_per_lane 0 or 1 (got %d)", ppl);
   StepArgs<R> a;
   fill_common<R>(c, a);
   for (const auto &in : c->inst)
@@ -2496,8 +2496,7 @@ emcgpu_status emcgpu_autotune(emcgpu_ctx *c, emcgpu_autotune_args *t) {
   if (c->n_baths > 0)
     return fail(c, EMCGPU_ERR_STATE, "autotune is not available with phonon baths");
   if (c->track_pos)
-    return fail(c, EMCGPU_ERR_STATE, "autotune is not available with tracked positions "
-                                     "(one particle per lane)");
+    return fail(c, EMCGPU_ERR_STATE, "autotune is not available with tracked positions");
   // plasma screening updates q_s^2 and the screened tables after every
   // step; the trials would leave them at the state of the last trial step
   for (int i = 0; i < c->n_inst; i++)
