@@ -23,7 +23,7 @@
 
 namespace emcgpu {
 template <typename R>
-hipError_t launch_steps(const StepArgs<R> &a, int mode, int ppt, hipStream_t st);
+hipError_t launch_steps(const StepArgs<R> &a, int mode, int ppt, double events, hipStream_t st);
 template <typename R>
 hipError_t launch_init(const StepArgs<R> &a, double init_mean, double init_sigma, hipStream_t st);
 template <typename R>
@@ -890,10 +890,11 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
     return fail(c, EMCGPU_ERR_ARG, "tracked positions take particles_per_lane 0 or 1 (got %d)", ppl);
   StepArgs<R> a;
   fill_common<R>(c, a);
+  double events = 0.0;  // expected per particle and step, the most of any valley
   for (const auto &in : c->inst)
     for (size_t v = 0; in.count && v < in.table_mech.size(); v++)
       if (!in.table_mech[v].empty())
-        a.events = std::max(a.events, s->dt / in.tau0[v]);
+        events = std::max(events, s->dt / in.tau0[v]);
   if (baths) {
     a.tally = c->d_tally;
     a.tally_bins = c->tally_bins;
@@ -904,7 +905,7 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
           a.lds_win = std::max(a.lds_win, 2 * (in.total_bins + (int)in.baths.size()));
   }
   const int asked = ppl ? ppl : c->tuned_ppl;  // 0: left to the library
-  int ppt = replay ? 1 : fitting_ppt(a, asked ? asked : default_ppt(c, K == 1, a.events));
+  int ppt = replay ? 1 : fitting_ppt(a, asked ? asked : default_ppt(c, K == 1, events));
   long long max_count = 0;
   for (const auto &in : c->inst)
     max_count = std::max<long long>(max_count, (long long)in.count);
@@ -947,7 +948,7 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
     if (reserve_only) {
       // a later call of one step may take fewer particles per lane
       if (!replay && !asked) {
-        shape(fitting_ppt(a, default_ppt(c, true, a.events)));
+        shape(fitting_ppt(a, default_ppt(c, true, events)));
         if ((st = ensure_partial(c, 1, n_tiles)) || (st = ensure_chunks(c, 1, n_chunks)))
           return st;
       }
@@ -1059,7 +1060,7 @@ emcgpu_status run_steps(emcgpu_ctx *c, const emcgpu_step_args *s,
     }
     if (s->timing)
       HIPCHK_CLEAN(hipEventRecord(c->ev0, c->stream));
-    HIPCHK_CLEAN(launch_steps<R>(a, replay ? 1 : 0, ppt, c->stream));
+    HIPCHK_CLEAN(launch_steps<R>(a, replay ? 1 : 0, ppt, events, c->stream));
     if (s->timing) {
       HIPCHK_CLEAN(hipEventRecord(c->ev1, c->stream));
       HIPCHK_CLEAN(hipEventSynchronize(c->ev1));

@@ -257,7 +257,6 @@ struct StepArgs {
   // parameters that any instance uses, tallies and window sums, each wave's
   // particles and sums (set by the launch)
   int lds_params, lds_hot, lds_wave;
-  double events;  // expected scatter events per particle and step (most of any valley)
 };
 
 // LDS of one workgroup (160 KB per CU on gfx950)

@@ -1,14 +1,16 @@
 // emcgpu_kernels.hip -- gfx950 kernels of the EMC particle step.
 //
-// A wave owns 64 * PPT particles and keeps them in LDS for all steps fused
-// into a launch, so HBM sees the SoA state once per launch.  Each step is the free-flight / scatter loop of
-// basicBulkParticleHandler::moveParticles
+// A wave owns 64 * PPT particles and keeps them on the chip for all steps fused
+// into a launch, so HBM sees the SoA state once per launch: in LDS
+// (k_bulk_fused), or, where a launch has one or a few steps, in registers
+// (k_bulk_lanes) or streamed through (k_bulk_once).  Each step is the
+// free-flight / scatter loop of basicBulkParticleHandler::moveParticles
 // (examples/bulkSimulation/basicBulkParticleHandler.hpp:195-221):
 //   drift min(tau, dt); while (dt - tau > 0) { scatter; tau += tau';
 //   drift min(rem, tau'); rem -= tau' }; tau -= dt
 // followed by the per-step ensemble sums (FP64 per lane, wave reductions,
-// one FP64 partial per wave per step, combined by the compensated two-pass
-// reduction k_reduce_chunks / k_reduce_final).
+// one FP64 partial per wave per step, combined by the compensated reduction
+// k_reduce_chunks, with k_reduce_final where there are several chunks).
 //
 // Random numbers:
 //   production: Philox-4x32-10 keyed by the seed, counter
@@ -220,9 +222,10 @@ __device__ __forceinline__ void tally_flush(const InstDev<R> *P, const uint32_t 
 // steps are held in LDS
 constexpr int kRing = 8;
 // a pass is run while this many particles have an event pending (a wave has
-// 64 lanes); fewer wait for the next step's.  10M Si FP32 / 4M two-valley
-// FP64, ms: 8 pending 3.08 / 0.76, 16 2.91 / 0.69, 24 to 32 2.90 / 0.68,
-// 48 2.96 / 0.70, 64 3.59 / 0.71
+// 64 lanes); fewer wait for the next step's.  us per step, 10M Si FP32 (64
+// steps) / 4M two-valley FP64 (16 steps): 8 pending 42.3 / 37.3, 16 40.5 /
+// 34.4, 24 40.1 / 33.4, 28 40.3 / 33.6, 32 39.8 / 33.4, 40 40.0 / 33.4, 48
+// 40.7 / 33.4, 64 48.1 / 33.5
 constexpr int kPass = 28;
 // valley/subvalley word in LDS: not with its home lane, in step at kAtShift
 constexpr uint32_t kAway = 0x80000000u;
@@ -336,7 +339,8 @@ __device__ __forceinline__ void wave_lds_fence() {
 
 // waves per SIMD that the registers leave room for: as many as the LDS does in
 // the large ensembles (FP64 two-valley: 173 VGPRs allow two waves, 168 three,
-// 0.68 -> 0.57 ms)
+// 0.68 -> 0.57 ms with the 16 VGPRs that it then spills, four per lane; 2 to 24
+// in the other FP64 kernels)
 template <typename R, int PPT, bool HOT, bool POS, int NV>
 __global__ __launch_bounds__(kTile, PPT == 1 ? 1 : sizeof(R) == 8 ? 3 : 6) void k_bulk_fused(StepArgs<R> a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -1944,8 +1948,9 @@ size_t once_lds(StepArgs<R> &a) {
 //   positions (8M FP64: 283 / 358)
 // - one step with positions of one valley, two per lane (k_bulk_once spills):
 //   300k FP32 20.3 / 21.0
+// events: expected per particle and step
 template <typename R>
-bool keeps_lanes(const StepArgs<R> &a, int ppt) {
+bool keeps_lanes(const StepArgs<R> &a, int ppt, double events) {
   const bool fp64 = sizeof(R) == 8;
   if (ppt == 1) {
     if (a.n_steps <= 4)
@@ -1962,11 +1967,11 @@ bool keeps_lanes(const StepArgs<R> &a, int ppt) {
     return a.px && ppt == 2;
   if (a.px || (!fp64 && ppt == 2))
     return true;
-  return a.events < 0.05 && (ppt == 4 || (long long)a.n_tiles * kSubs <= 8192);
+  return events < 0.05 && (ppt == 4 || (long long)a.n_tiles * kSubs <= 8192);
 }
 
 template <typename R, int PPT, bool HOT, bool POS>
-hipError_t launch_fused(StepArgs<R> a, hipStream_t st) {
+hipError_t launch_fused(StepArgs<R> a, double events, hipStream_t st) {
   size_t lds = fused_lds<R, PPT, POS>(a);
   const void *f = a.max_v == 1 ? (const void *)k_bulk_fused<R, PPT, HOT, POS, 1>
                                : (const void *)k_bulk_fused<R, PPT, HOT, POS, kMaxV>;
@@ -1976,7 +1981,7 @@ hipError_t launch_fused(StepArgs<R> a, hipStream_t st) {
       f = (const void *)k_bulk_once<R, PPT, HOT>;
     }
   }
-  if (keeps_lanes(a, PPT)) {
+  if (keeps_lanes(a, PPT, events)) {
     lds = (size_t)a.lds_params + a.lds_hot;
     if constexpr (PPT == 1 || (PPT == 2 && POS))
       if (a.max_v == 1)
@@ -2000,7 +2005,7 @@ hipError_t launch_fused(StepArgs<R> a, hipStream_t st) {
 }
 
 template <typename R, bool HOT>
-hipError_t launch_steps_t(const StepArgs<R> &a, int mode, int ppt, hipStream_t st) {
+hipError_t launch_steps_t(const StepArgs<R> &a, int mode, int ppt, double events, hipStream_t st) {
   if (mode == 1) {
     // tallies, then (8-byte aligned) the staged window sums
     const dim3 g(a.n_tiles), b(kTile);
@@ -2016,36 +2021,36 @@ hipError_t launch_steps_t(const StepArgs<R> &a, int mode, int ppt, hipStream_t s
   if (a.px) {  // positions tracked
     switch (ppt) {
     case 1:
-      return launch_fused<R, 1, HOT, true>(a, st);
+      return launch_fused<R, 1, HOT, true>(a, events, st);
     case 2:
-      return launch_fused<R, 2, HOT, true>(a, st);
+      return launch_fused<R, 2, HOT, true>(a, events, st);
     case 4:
-      return launch_fused<R, 4, HOT, true>(a, st);
+      return launch_fused<R, 4, HOT, true>(a, events, st);
     default:
       return hipErrorInvalidValue;
     }
   }
   switch (ppt) {
   case 1:
-    return launch_fused<R, 1, HOT, false>(a, st);
+    return launch_fused<R, 1, HOT, false>(a, events, st);
   case 2:
-    return launch_fused<R, 2, HOT, false>(a, st);
+    return launch_fused<R, 2, HOT, false>(a, events, st);
   case 4:
-    return launch_fused<R, 4, HOT, false>(a, st);
+    return launch_fused<R, 4, HOT, false>(a, events, st);
   case 8:
-    return launch_fused<R, 8, HOT, false>(a, st);
+    return launch_fused<R, 8, HOT, false>(a, events, st);
   default:
     return hipErrorInvalidValue;
   }
 }
 
 template <typename R>
-hipError_t launch_steps(const StepArgs<R> &a, int mode, int ppt, hipStream_t st) {
+hipError_t launch_steps(const StepArgs<R> &a, int mode, int ppt, double events, hipStream_t st) {
   if (a.n_tiles <= 0)
     return hipSuccess;
   if (extended(a))
-    return launch_steps_t<R, true>(a, mode, ppt, st);
-  return launch_steps_t<R, false>(a, mode, ppt, st);
+    return launch_steps_t<R, true>(a, mode, ppt, events, st);
+  return launch_steps_t<R, false>(a, mode, ppt, events, st);
 }
 
 template <typename R>
@@ -2108,8 +2113,8 @@ hipError_t launch_reduce(const double *partial, int n_steps, int n_tiles, int n_
   return hipGetLastError();
 }
 
-template hipError_t launch_steps<float>(const StepArgs<float> &, int, int, hipStream_t);
-template hipError_t launch_steps<double>(const StepArgs<double> &, int, int, hipStream_t);
+template hipError_t launch_steps<float>(const StepArgs<float> &, int, int, double, hipStream_t);
+template hipError_t launch_steps<double>(const StepArgs<double> &, int, int, double, hipStream_t);
 template hipError_t launch_observe<float>(const StepArgs<float> &, hipStream_t);
 template hipError_t launch_observe<double>(const StepArgs<double> &, hipStream_t);
 template hipError_t launch_init<float>(const StepArgs<float> &, double, double, hipStream_t);
