@@ -209,3 +209,26 @@ def test_two_threads_with_workgroups_of_different_lds():
         (p, obs), (q, want) = together[name], alone[name]
         assert all(np.array_equal(p[key], q[key]) for key in p)
         assert np.array_equal(obs, want)
+
+
+def test_reserve_covers_a_shorter_call():
+    """positions in FP64: two steps take four particles per lane, one step
+    takes one and four times the partials.  A context that reserved two steps
+    runs one without taking device memory"""
+    import torch
+    from viennaemc_amd import emcgpu
+    spec, n, used = MODELS["si_jacoboni"], 4_000_000, []
+    for _ in range(2):  # the first context also loads the kernels
+        ctx = emcgpu.Context(precision=emcgpu.FP64)
+        ctx.setup(0, spec)
+        ctx.resize([n])
+        ctx.set_box(0, (3e-7, 2e-7, 4e-7))
+        ctx.init_particles(0, 2, spec["T"])
+        ctx.reserve(1e-15, 2)
+        ctx.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        ctx.step(1e-15, 1, seed=3)
+        ctx.synchronize()
+        used.append(free - torch.cuda.mem_get_info()[0])
+        ctx.close()
+    assert used[1] <= 0
