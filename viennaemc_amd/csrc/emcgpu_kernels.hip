@@ -1937,9 +1937,9 @@ size_t once_lds(StepArgs<R> &a) {
 //   4.5 / 5.0; 8M FP64: si 313 / 368, 214 / 230, tv 279 / 447, 176 / 231; a tie
 //   at 4 steps of tv in FP32 (1M: 13.9 / 13.9).  Where the waves fill the chip
 //   and the registers of k_bulk_fused leave two waves per SIMD, longer ones
-//   too: FP64 tv to 32 steps (8M: 148 / 161; 64 the other way round); with
-//   positions any number (1M si, 64 steps: FP64 30.4 / 38.0, FP32 12.6 / 13.8;
-//   FP32 tv to 8: 13.6 / 13.7)
+//   too: FP64 tv to 32 steps (8M: 148 / 161; where events are frequent a tie by
+//   then, 10 fs 279 / 282, 1M 38.2 / 37.4); with positions any number (1M si, 64
+//   steps: FP64 30.4 / 38.0, FP32 12.6 / 13.8; FP32 tv to 8: 13.6 / 13.7)
 // - one step of two or four per lane, several valleys: while events are rare
 //   (at 0.044 expected per particle 4M FP64 100 / 102, 10M 279 / 305, 8M FP32
 //   74 / 84; at 0.088 4M FP64 112 / 109; with baths at 0.2 204 / 170 at 1M;
