@@ -215,8 +215,16 @@ def test_reserve_covers_a_shorter_call():
     """positions in FP64: two steps take four particles per lane, one step
     takes one and four times the partials.  A context that reserved two steps
     runs one without taking device memory"""
-    import torch
+    import ctypes as C
+    from test_zz_no_alloc import _hip
     from viennaemc_amd import emcgpu
+    hip = _hip()  # the runtime that the library is linked against
+
+    def free_bytes():
+        free, total = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
     spec, n, used = MODELS["si_jacoboni"], 4_000_000, []
     for _ in range(2):  # the first context also loads the kernels
         ctx = emcgpu.Context(precision=emcgpu.FP64)
@@ -226,9 +234,9 @@ def test_reserve_covers_a_shorter_call():
         ctx.init_particles(0, 2, spec["T"])
         ctx.reserve(1e-15, 2)
         ctx.synchronize()
-        free = torch.cuda.mem_get_info()[0]
+        free = free_bytes()
         ctx.step(1e-15, 1, seed=3)
         ctx.synchronize()
-        used.append(free - torch.cuda.mem_get_info()[0])
+        used.append(free - free_bytes())
         ctx.close()
     assert used[1] <= 0
